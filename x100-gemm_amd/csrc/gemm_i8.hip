@@ -4,16 +4,16 @@
 // that falls back to the scalar gemm_ref_i8 (src/gemm_ref.c:17-26).  Integer arithmetic is exact,
 // so every kernel here is bit-identical to gemm_ref_i8 for any K below 2^17 (|sum| < 2^31).
 //
-// Three kernels:
-//   k_gemm_mfma    tiled MFMA kernel (v_mfma_i32_32x32x32_i8).  A tiles go to LDS row-major with
-//                  an XOR swizzle on 16-byte chunks; B tiles are transposed in registers
-//                  (v_perm_b32) into "k-quad" dwords (4 consecutive k of one column) so that both
-//                  MFMA operands are k-contiguous.  Double-buffered LDS, C loaded into the
-//                  accumulators (C += A.B), XCD-aware grouped tile order.
-//   k_gemm_skinny  M <= 16 rows (speculative-verify shapes): HBM-bound on B.  Split-K over
-//                  256-row chunks, B streamed once through LDS, dot4 on transposed k-quads,
-//                  int32 atomics into C (exact and order independent).
-//   k_gemm_generic any shape / alignment (byte loads); correctness fallback.
+// Kernels (x100_gemm_i8_launch picks one by sizes and alignment):
+//   k_gemm_big     256x256 tiles, M and N multiples of 256: direct global->LDS DMA, transposing LDS
+//                  reads for B, v_mfma_i32_32x32x32_i8.
+//   k_gemm_tile    tiles from 32x32 to 128x128 for every other shape and alignment, same operand
+//                  path in a 4-slot ring of 128-k stages (unaligned operands through registers).
+//   k_gemm_skinny  M <= 16 rows (speculative-verify shapes): HBM-bound on B.  Split-K, B streamed
+//   (_mfma)        once through LDS, int32 atomics into C (exact and order independent).
+//   k_gemm_generic byte loads and scalar products: operands under 16 bytes, rows of 2^24 and more.
+#include <math.h>
+
 #include <type_traits>
 
 #include "x100_common.h"
@@ -28,8 +28,8 @@ constexpr int BK = 64;  // k bytes per pipeline stage
 // tiles of one XCD share A row panels and B column panels in its L2.
 X100_DEV void tile_coords(int bid, int nblk, int tiles_m, int tiles_n, int &tm, int &tn)
 {
-    int t = bid;
-    if ((nblk & 7) == 0) t = (bid & 7) * (nblk >> 3) + (bid >> 3);
+    const int x = bid & 7, q = nblk >> 3;
+    const int t = x * q + min(x, nblk & 7) + (bid >> 3);
     constexpr int GROUP_M = 4;
     int per_group = GROUP_M * tiles_n;
     int g = t / per_group;
@@ -38,156 +38,6 @@ X100_DEV void tile_coords(int bid, int nblk, int tiles_m, int tiles_n, int &tm, 
     int r = t - g * per_group;
     tm = first_m + r % gsize;
     tn = r / gsize;
-}
-
-// A tile in LDS: BM rows x 64 bytes; 16-byte chunk c of row r stored at chunk c ^ ((r>>1)&3)
-// so that 8 consecutive lanes reading one chunk column hit 8 distinct 16-byte bank groups.
-X100_DEV int a_lds_off(int r, int c) { return r * BK + ((c ^ ((r >> 1) & 3)) << 4); }
-
-template <int FM, int FN, int WM, int WN, bool EDGE, bool ACC>
-__global__ __launch_bounds__(WM *WN * 64) void k_gemm_mfma(int M, int N, int K,
-                                                           const int8_t *__restrict__ A,
-                                                           const int8_t *__restrict__ B,
-                                                           int32_t *__restrict__ C, int tiles_m,
-                                                           int tiles_n)
-{
-    constexpr int NT = WM * WN * 64;
-    constexpr int BM = WM * FM * 32;
-    constexpr int BN = WN * FN * 32;
-    constexpr int A_IT = BM * 4 / NT;             // 16-byte A chunks per thread per stage
-    constexpr int B_UNITS = BN;                   // (k-quad, 16 columns) units per stage
-    constexpr int B_IT = (B_UNITS + NT - 1) / NT;
-    static_assert(A_IT * NT == BM * 4, "A tile must split evenly over the threads");
-
-    __shared__ __attribute__((aligned(16))) int8_t As[2][BM * BK];
-    __shared__ __attribute__((aligned(16))) uint32_t Bs[2][16 * BN];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WN, wn = wave % WN;
-    const int lcol = lane & 31, lgrp = lane >> 5;
-    int tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN;
-    // EDGE = false is only launched when M % BM == 0, N % BN == 0 and K % BK == 0.
-    const bool full_mn = !EDGE || ((m0 + BM <= M) && (n0 + BN <= N));
-
-    // Accumulators start from C (ACC: C += A.B) or from zero (C = A.B, C never read).  32x32 MFMA
-    // output layout: lane l, register r holds row 8*(r/4) + 4*(l/32) + r%4, column l%32.
-    v16i acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int gn = n0 + wn * FN * 32 + 32 * j + lcol;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int gm = m0 + wm * FM * 32 + 32 * i + 8 * (r >> 2) + 4 * lgrp + (r & 3);
-                acc[i][j][r] = (ACC && (full_mn || (gm < M && gn < N))) ? C[(size_t)gm * N + gn] : 0;
-            }
-        }
-
-    v4i ra[A_IT];
-    v4i rb[B_IT][4];
-
-    auto gload = [&](int kt) {
-        const int k0 = kt * BK;
-        const bool full = !EDGE || (full_mn && (k0 + BK <= K));
-#pragma unroll
-        for (int p = 0; p < A_IT; p++) {
-            const int ch = tid + p * NT, r = ch >> 2, c = ch & 3;
-            const int gm = m0 + r, gk = k0 + 16 * c;
-            if (full || (gm < M && gk < K))
-                ra[p] = *(const v4i *)(A + (size_t)gm * K + gk);
-            else
-                ra[p] = v4i{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int p = 0; p < B_IT; p++) {
-            const int u = tid + p * NT;
-            if (B_UNITS % NT == 0 || u < B_UNITS) {
-                const int kq = u / (BN / 16), nc = u % (BN / 16);
-                const int gn = n0 + 16 * nc;
-#pragma unroll
-                for (int rr = 0; rr < 4; rr++) {
-                    const int gk = k0 + 4 * kq + rr;
-                    if (full || (gk < K && gn < N))
-                        rb[p][rr] = *(const v4i *)(B + (size_t)gk * N + gn);
-                    else
-                        rb[p][rr] = v4i{0, 0, 0, 0};
-                }
-            }
-        }
-    };
-
-    auto lstore = [&](int buf) {
-#pragma unroll
-        for (int p = 0; p < A_IT; p++) {
-            const int ch = tid + p * NT, r = ch >> 2, c = ch & 3;
-            *(v4i *)(&As[buf][a_lds_off(r, c)]) = ra[p];
-        }
-#pragma unroll
-        for (int p = 0; p < B_IT; p++) {
-            const int u = tid + p * NT;
-            if (B_UNITS % NT == 0 || u < B_UNITS) {
-                const int kq = u / (BN / 16), nc = u % (BN / 16);
-                uint32_t o[16];
-#pragma unroll
-                for (int cg = 0; cg < 4; cg++)
-                    transpose4x4((uint32_t)rb[p][0][cg], (uint32_t)rb[p][1][cg],
-                                 (uint32_t)rb[p][2][cg], (uint32_t)rb[p][3][cg], o[4 * cg + 0],
-                                 o[4 * cg + 1], o[4 * cg + 2], o[4 * cg + 3]);
-                v4u *dst = (v4u *)(&Bs[buf][kq * BN + 16 * nc]);
-                dst[0] = v4u{o[0], o[1], o[2], o[3]};
-                dst[1] = v4u{o[4], o[5], o[6], o[7]};
-                dst[2] = v4u{o[8], o[9], o[10], o[11]};
-                dst[3] = v4u{o[12], o[13], o[14], o[15]};
-            }
-        }
-    };
-
-    const int nk = (K + BK - 1) / BK;
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (int kt = 0; kt < nk; kt++) {
-        const int buf = kt & 1;
-        if (kt + 1 < nk) gload(kt + 1);
-#pragma unroll
-        for (int kk = 0; kk < 2; kk++) {
-            v4i af[FM], bf[FN];
-#pragma unroll
-            for (int i = 0; i < FM; i++) {
-                const int r = wm * FM * 32 + 32 * i + lcol;
-                af[i] = *(const v4i *)(&As[buf][a_lds_off(r, 2 * kk + lgrp)]);
-            }
-#pragma unroll
-            for (int j = 0; j < FN; j++) {
-                const int n = wn * FN * 32 + 32 * j + lcol;
-                const int kq = 8 * kk + 4 * lgrp;
-                const uint32_t *bp = &Bs[buf][kq * BN + n];
-                bf[j] = v4i{(int)bp[0], (int)bp[BN], (int)bp[2 * BN], (int)bp[3 * BN]};
-            }
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int j = 0; j < FN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-        if (kt + 1 < nk) lstore(buf ^ 1);
-        __syncthreads();
-    }
-
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int gn = n0 + wn * FN * 32 + 32 * j + lcol;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int gm = m0 + wm * FM * 32 + 32 * i + 8 * (r >> 2) + 4 * lgrp + (r & 3);
-                if (full_mn || (gm < M && gn < N)) C[(size_t)gm * N + gn] = acc[i][j][r];
-            }
-        }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -653,6 +503,374 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_big(int M, int N, int K, const
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// k_gemm_tile: output tiles below 256 x 256, any M and N.  Tile WM*FM*32 rows x WN*FN*32 columns on
+// WM*WN*KW waves; each of the KW wave groups takes 1/KW of every K stage and the groups' sums are
+// added through LDS at the end, so that a product with few tiles still runs 4 waves per tile.
+//
+// * K stages of 128: A rows are whole 128-byte cache lines, B 128 k-rows x BN bytes.  LDS chunks
+//   swizzled like k_gemm_big's (tile_a_pos, tile_b_pos): ds_read_b128 for A, ds_read_b64_tr_b8 for B,
+//   both conflict-free, B with no register transpose.
+// * ALN (K, N multiples of 16, A and B 16-byte aligned): the stages reach LDS by global->LDS DMA
+//   through a ring of S slots, S - 1 of them in flight.  Rows, columns and k past the end read the
+//   last valid chunk (never another address); A's k past K is cleared in registers.
+// * otherwise: 16-byte loads at any byte address (gfx950 global loads need no alignment) into
+//   registers, PD stages ahead, then ds_write to the same layout.  A chunk that would cross the end
+//   of the matrix is loaded from its last 16 bytes and shifted down, so nothing past it is read.
+// * The loop is short per stage, so its fixed cost decides: the next stage's fragments are read while
+//   the current one's MFMAs run, one barrier per stage and no LDS wait at it, and (ALN) a turn of the
+//   ring is unrolled so that slots, waits and LDS addresses are constants (1024 x 1024 x 4096 on
+//   64 x 64 tiles: 17.5 us with fragments read and used in the same stage, 13.1, 11.9, 10.7).
+// * C is read (ACC) first and written as dwords (32 lanes = one 128-byte row segment): any alignment.
+// Bound by operand delivery (L2 to LDS, 12-16 TB/s over the chip) with many tiles and by the stage's
+// latency with few.  In place of register-staged 64-k tiles and of scalar products on unaligned
+// shapes: 333 x 6144 x 2048 26.7 -> 11.7 us, 2048^3 24.3 -> 15.0, 1001 x 1503 x 999 178 -> 10.3.
+// ------------------------------------------------------------------------------------------------
+typedef int v4i_u __attribute__((ext_vector_type(4), aligned(1)));
+
+X100_DEV int tile_a_pos(int r, int c) { return c ^ ((r >> 1) & 7); }
+// B rows of BN bytes: 32 lanes of a transposing read take the chunk pair (c, c ^ 1) of 8 consecutive
+// k-rows, 16 granules that must fall on distinct 16-byte columns of a 256-byte bank line; 256 / BN
+// rows share a line.
+template <int BN> X100_DEV int tile_b_pos(int k, int c) { return c ^ (2 * ((k / (256 / BN)) & (BN / 32 - 1))); }
+
+// v >> 8 s for s = 0 .. 15 bytes (zeros shifted in).
+X100_DEV v4i shr_bytes(v4i v, int s)
+{
+    const uint64_t lo = (uint64_t)(uint32_t)v[0] | (uint64_t)(uint32_t)v[1] << 32;
+    const uint64_t hi = (uint64_t)(uint32_t)v[2] | (uint64_t)(uint32_t)v[3] << 32;
+    const int b = 8 * (s & 7);
+    const uint64_t l1 = b ? (lo >> b) | (hi << (64 - b)) : lo, h1 = hi >> b;
+    const uint64_t l = s < 8 ? l1 : h1, h = s < 8 ? h1 : 0;
+    return v4i{(int)(uint32_t)l, (int)(uint32_t)(l >> 32), (int)(uint32_t)h, (int)(uint32_t)(h >> 32)};
+}
+// The first n bytes of v (n <= 0: none; n >= 16: all), zeros after.
+X100_DEV v4i keep_bytes(v4i v, int n)
+{
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        const int nb = n - 4 * d;
+        v[d] = nb >= 4 ? v[d] : nb <= 0 ? 0 : (v[d] & (int)((1u << (8 * nb)) - 1));
+    }
+    return v;
+}
+
+template <int WM, int WN, int FM, int FN, int KW, int S, bool ALN, bool ACC>
+__global__ __launch_bounds__(WM *WN *KW * 64, WM *WN *KW <= 4 || WM *WN *FM *FN >= 8 ? 2 : 3) void k_gemm_tile(int M, int N, int K, const int8_t *__restrict__ A,
+                                                            const int8_t *__restrict__ B, int32_t *__restrict__ C,
+                                                            int tiles_m, int tiles_n)
+{
+    constexpr int NW = WM * WN * KW, NT = NW * 64, BM = WM * FM * 32, BN = WN * FN * 32;
+    constexpr int A_IT = BM * 8 / NT, B_IT = BN * 8 / NT, OPS = A_IT + B_IT;   // 16-byte chunks per lane and stage
+    constexpr int ASZ = BM * 128, STAGE = ASZ + 128 * BN, CPB = BN / 16;
+    static_assert(A_IT * NT == BM * 8 && B_IT * NT == BN * 8, "a stage splits evenly over the threads");
+    static_assert(!ALN || S == 4, "the ring of the aligned form");
+    static_assert(KW == 1 || S * STAGE >= NW * FM * FN * 4096, "the partial sums must fit the ring");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[S * STAGE];
+
+    const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+    const int kw = w / (WM * WN), wm = w / WN % WM, wn = w % WN;
+    const int lcol = lane & 31, lgrp = lane >> 5;
+    int tm, tn;
+    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int nk = (K + 127) / 128;
+    const bool full = m0 + BM <= M && n0 + BN <= N;
+
+    // Chunk p of this lane: linear index (p NW + w) 64 + lane of the operand's stage.
+    auto a_row = [&](int p) __attribute__((always_inline)) { return ((p * NW + w) * 64 + lane) >> 3; };
+    auto a_col = [&](int p) __attribute__((always_inline)) {
+        const int r = a_row(p);
+        return 16 * tile_a_pos(r, lane & 7);
+    };
+    auto b_row = [&](int p) __attribute__((always_inline)) { return ((p * NW + w) * 64 + lane) / CPB; };
+    auto b_col = [&](int p) __attribute__((always_inline)) {
+        const int k = b_row(p);
+        return 16 * tile_b_pos<BN>(k, lane % CPB);
+    };
+
+    // C of the registers this wave stores, read before anything else so that the loads, the oldest,
+    // never hold up a stage's wait, and added after the K loop.
+    v16i acc[FM][FN];
+    int cp[FM][FN][16 / KW];
+    // element offset in the tile's C of row 8 (r / 4) + 4 lgrp + r % 4 of fragment (i, j)
+    int32_t *Ct = C + (size_t)m0 * N + n0;
+    const int mr = M - m0, nr = N - n0;   // rows and columns left
+    auto c_row = [&](int i, int r) __attribute__((always_inline)) {
+        return wm * FM * 32 + 32 * i + 8 * (r >> 2) + 4 * lgrp + (r & 3);
+    };
+    auto c_col = [&](int j) __attribute__((always_inline)) { return wn * FN * 32 + 32 * j + lcol; };
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            acc[i][j] = v16i{};
+            // unconditional: past the edge the last row or column, not stored (a branch per load
+            // cost 4 us at 2048^3)
+#pragma unroll
+            for (int r = 0; r < 16 / KW; r++)
+                cp[i][j][r] = ACC ? Ct[(uint32_t)min(c_row(i, 16 / KW * kw + r), mr - 1) * (uint32_t)N + (uint32_t)min(c_col(j), nr - 1)] : 0;
+        }
+    // Fragments of one stage (LDS at st) and their products; the last stage's A is cleared past K.
+    // Two sets: the next stage's reads are in flight while the current one's MFMAs run.
+    constexpr int KS = 4 / KW;   // 32-k steps per wave and stage
+    struct Frags {
+        v4i a[KS][FM], b[KS][FN];
+    };
+    auto read = [&](Frags &f, const uint8_t *st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < KS; t++) {
+            const int ks = kw * KS + t;
+#pragma unroll
+            for (int i = 0; i < FM; i++) {
+                const int r = wm * FM * 32 + 32 * i + lcol;
+                f.a[t][i] = *(const v4i *)(st + r * 128 + 16 * tile_a_pos(r, 2 * ks + lgrp));
+            }
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                const int c = 2 * (wn * FN + j) + ((lane >> 4) & 1);
+                const int k0 = 32 * ks + 16 * lgrp + ((lane & 15) >> 1), k1 = k0 + 8;
+                const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                    (lds_v2i *)(const lds_u8 *)(st + ASZ + k0 * BN + 16 * tile_b_pos<BN>(k0, c) + 8 * (lane & 1)));
+                const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                    (lds_v2i *)(const lds_u8 *)(st + ASZ + k1 * BN + 16 * tile_b_pos<BN>(k1, c) + 8 * (lane & 1)));
+                f.b[t][j] = v4i{lo.x, lo.y, hi.x, hi.y};
+            }
+        }
+    };
+    auto mma = [&](Frags &f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < KS; t++)
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[t][i], f.b[t][j], acc[i][j], 0, 0, 0);
+    };
+    auto mma_last = [&](Frags &f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < KS; t++)
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+                f.a[t][i] = keep_bytes(f.a[t][i], K - ((nk - 1) * 128 + 32 * (kw * KS + t) + 16 * lgrp));
+        mma(f);
+    };
+    Frags f0, f1;
+
+    if constexpr (ALN) {
+        const uint32_t sbase = lds_addr(smem);
+        uint32_t aoff[A_IT], boff[B_IT];
+#pragma unroll
+        for (int p = 0; p < A_IT; p++) aoff[p] = (uint32_t)min(a_row(p), M - 1 - m0) * (uint32_t)K + a_col(p);
+#pragma unroll
+        for (int p = 0; p < B_IT; p++) boff[p] = (uint32_t)b_row(p) * (uint32_t)N + min(b_col(p), N - 16 - n0);
+        // the next stage to request: its operands and ring slot
+        const int8_t *ak = A + (size_t)m0 * K, *bk = B + n0;
+        const size_t bstep = (size_t)128 * N;
+        // a full stage into slot; then the next one
+        auto issue_full = [&](int slot) __attribute__((always_inline)) {
+            const uint32_t sb = sbase + (uint32_t)(slot * STAGE) + 1024u * w;
+#pragma unroll
+            for (int p = 0; p < A_IT; p++) dma16s(aoff[p], ak, __builtin_amdgcn_readfirstlane(sb + 1024u * NW * p));
+#pragma unroll
+            for (int p = 0; p < B_IT; p++) dma16s(boff[p], bk, __builtin_amdgcn_readfirstlane(sb + ASZ + 1024u * NW * p));
+            ak += 128;
+            bk += bstep;
+        };
+        // stage kt; k past K: the last valid chunk of A's row, the last row of B
+        auto issue = [&](int kt) __attribute__((always_inline)) {
+            const int kr = K - kt * 128;
+            if (kr >= 128) {
+                issue_full(kt & (S - 1));
+            } else {   // kr is a multiple of 16
+                const uint32_t sb = sbase + (uint32_t)((kt & (S - 1)) * STAGE) + 1024u * w;
+#pragma unroll
+                for (int p = 0; p < A_IT; p++)
+                    dma16s(aoff[p] - a_col(p) + min(a_col(p), kr - 16), ak,
+                           __builtin_amdgcn_readfirstlane(sb + 1024u * NW * p));
+#pragma unroll
+                for (int p = 0; p < B_IT; p++)
+                    dma16s(boff[p] - (uint32_t)max(b_row(p) - (kr - 1), 0) * (uint32_t)N, bk,
+                           __builtin_amdgcn_readfirstlane(sb + ASZ + 1024u * NW * p));
+            }
+        };
+#pragma unroll
+        for (int t = 0; t < S - 1; t++)
+            if (t < nk) issue(t);
+        // Wait for a stage with up to n younger stages outstanding.  The barrier makes it every
+        // wave's.  No wait for LDS reads: the ones still in flight are of the stage before, whose slot
+        // is refilled only after the next barrier, which each wave passes with its products of that
+        // stage, and so the reads, done.
+        auto landed = [&](int n) __attribute__((always_inline)) {
+            if (n >= 2) wait_vmcnt<2 * OPS>();
+            else if (n == 1) wait_vmcnt<OPS>();
+            else wait_vmcnt<0>();
+            asm volatile("s_barrier" ::: "memory");
+        };
+        // fragments of stage kt in f; stage kt + 1 is read into g while they are multiplied, stage
+        // kt + S - 1 requested into the slot of stage kt - 1
+        auto step = [&](int kt, Frags &f, Frags &g) __attribute__((always_inline)) {
+            landed(min(S - 3, nk - 2 - kt));
+            read(g, smem + ((kt + 1) & (S - 1)) * STAGE);
+            if (kt + S - 1 < nk) issue(kt + S - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mma(f);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        landed(min(S - 2, nk - 1));
+        read(f0, smem);
+        int kt = 0;
+        // whole stages, a turn of the ring at a time: slots, waits and LDS addresses are constants
+        for (; kt + 2 * S - 2 < nk - 1; kt += S)
+            static_for<S>([&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                Frags &f = i & 1 ? f1 : f0, &g = i & 1 ? f0 : f1;
+                landed(S - 3);
+                read(g, smem + ((i + 1) & (S - 1)) * STAGE);
+                issue_full((i + S - 1) & (S - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                mma(f);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        for (; kt + 2 < nk; kt += 2) {
+            step(kt, f0, f1);
+            step(kt + 1, f1, f0);
+        }
+        if (kt + 1 < nk) {
+            step(kt, f0, f1);
+            mma_last(f1);
+        } else {
+            mma_last(f0);
+        }
+    } else {
+        constexpr int PD = 2;   // stages held in registers
+        static_assert(S == 2, "two LDS slots");
+        // chunk offsets from the tile's first row (column) and the stage's first k
+        uint32_t aoff[A_IT], boff[B_IT];
+#pragma unroll
+        for (int p = 0; p < A_IT; p++) aoff[p] = (uint32_t)a_row(p) * (uint32_t)K + a_col(p);
+#pragma unroll
+        for (int p = 0; p < B_IT; p++) boff[p] = (uint32_t)b_row(p) * (uint32_t)N + b_col(p);
+        const size_t alim = (size_t)M * K - 16, blim = (size_t)K * N - 16;   // last chunk inside the matrix
+        v4i ra[PD][A_IT], rb[PD][B_IT];
+        // Stage kt.  No offset passes the last chunk: rows, columns and k past the end read other valid
+        // bytes.
+        auto gload = [&](int kt, v4i(&va)[A_IT], v4i(&vb)[B_IT]) __attribute__((always_inline)) {
+            const size_t a0 = min((size_t)m0 * K + (size_t)kt * 128, alim), b0 = min((size_t)kt * 128 * N + n0, blim);
+            const uint32_t al = (uint32_t)min(alim - a0, (size_t)0xffffffffu), bl = (uint32_t)min(blim - b0, (size_t)0xffffffffu);
+#pragma unroll
+            for (int p = 0; p < A_IT; p++) va[p] = *(const v4i_u *)(A + a0 + min(aoff[p], al));
+#pragma unroll
+            for (int p = 0; p < B_IT; p++) vb[p] = *(const v4i_u *)(B + b0 + min(boff[p], bl));
+        };
+        // ds_write of stage kt; a chunk read from before its own offset is shifted down (only the last
+        // 16 bytes of the matrix: the last two stages)
+        auto lstore = [&](int kt, v4i(&va)[A_IT], v4i(&vb)[B_IT]) __attribute__((always_inline)) {
+            uint8_t *st = smem + (kt & 1) * STAGE + 16 * tid;
+            if (kt >= nk - 2) {
+                const size_t a0 = (size_t)m0 * K + (size_t)kt * 128, b0 = (size_t)kt * 128 * N + n0;
+#pragma unroll
+                for (int p = 0; p < A_IT; p++)
+                    va[p] = shr_bytes(va[p], a0 + aoff[p] > alim ? (int)min(a0 + aoff[p] - alim, (size_t)15) : 0);
+#pragma unroll
+                for (int p = 0; p < B_IT; p++)
+                    vb[p] = shr_bytes(vb[p], b0 + boff[p] > blim ? (int)min(b0 + boff[p] - blim, (size_t)15) : 0);
+            }
+#pragma unroll
+            for (int p = 0; p < A_IT; p++) *(v4i *)(st + 16 * NT * p) = va[p];
+#pragma unroll
+            for (int p = 0; p < B_IT; p++) *(v4i *)(st + ASZ + 16 * NT * p) = vb[p];
+        };
+        // stages 0 and 1 to LDS, stage 2 + i in register slot i
+        {
+            v4i a0[A_IT], b0[B_IT], a1[A_IT], b1[B_IT];
+            gload(0, a0, b0);
+            if (1 < nk) gload(1, a1, b1);
+#pragma unroll
+            for (int i = 0; i < PD; i++)
+                if (2 + i < nk) gload(2 + i, ra[i], rb[i]);
+            lstore(0, a0, b0);
+            if (1 < nk) lstore(1, a1, b1);
+        }
+        __syncthreads();
+        read(f0, smem);
+        // stage kt in f, stage kt + 1 in LDS, stage kt + 2 in slot i
+        auto step = [&](int kt, int i, Frags &f, Frags &g) __attribute__((always_inline)) {
+            __syncthreads();
+            read(g, smem + ((kt + 1) & 1) * STAGE);
+            if (kt + 2 < nk) {
+                lstore(kt + 2, ra[i], rb[i]);
+                if (kt + 2 + PD < nk) gload(kt + 2 + PD, ra[i], rb[i]);
+            }
+            mma(f);
+        };
+        int kt = 0;
+        for (; kt + PD < nk; kt += PD) {
+#pragma unroll
+            for (int i = 0; i < PD; i += 2) {
+                step(kt + i, i, f0, f1);
+                step(kt + i + 1, i + 1, f1, f0);
+            }
+        }
+        // nk - kt = 1 .. PD stages left
+#pragma unroll
+        for (int i = 0; i < PD; i++) {
+            if (kt + i + 1 < nk) {
+                if (i & 1) step(kt + i, i, f1, f0);
+                else step(kt + i, i, f0, f1);
+            } else if (kt + i + 1 == nk) {
+                if (i & 1) mma_last(f1);
+                else mma_last(f0);
+            }
+        }
+    }
+
+    if constexpr (KW > 1) {   // add the wave groups' sums; group kw finishes registers 16/KW kw .. of each fragment
+        lds_barrier();
+        int *red = (int *)smem;
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) red[(((w * FM + i) * FN + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 16 / KW; r++)
+#pragma unroll
+                    for (int v = 0; v < KW; v++)
+                        cp[i][j][r] += red[((((v * WM * WN + w % (WM * WN)) * FM + i) * FN + j) * 16 + 16 / KW * kw + r) * 64 + lane];
+    } else {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) cp[i][j][r] += acc[i][j][r];
+    }
+    // every sum is final before the first store: a wait for C between the stores would also wait
+    // for the stores before it
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int r = 0; r < 16 / KW; r++) asm volatile("" : "+v"(cp[i][j][r]));
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int r = 0; r < 16 / KW; r++) {
+                const int gm = c_row(i, 16 / KW * kw + r), gn = c_col(j);
+                if (full || (gm < mr && gn < nr)) Ct[(uint32_t)gm * (uint32_t)N + (uint32_t)gn] = cp[i][j][r];
+            }
+}
+
 // Skinny GEMM, M <= MR rows.  Block = W waves over columns [n0, n0+256) and k rows
 // [k0, k0+256); wave w owns rows k0 + RW*w .. +RW-1 (RW = 256/W).  Each lane streams RW/4 x 16
 // bytes of B (one 256-byte row slice per 16 lanes, fully coalesced), the wave stages its slice in
@@ -838,7 +1056,7 @@ __global__ __launch_bounds__(256) void k_gemm_skinny_mfma(int M, int N, int K, c
         }
 }
 
-// Generic fallback: 64x64 tile, 256 threads (4x4 outputs each), 32-deep byte tiles in LDS.
+// Any shape and alignment: 64x64 tile, 256 threads (4x4 outputs each), 32-deep byte tiles in LDS.
 // ACC: C += A.B; otherwise C = A.B (C not read).
 template <bool ACC>
 __global__ __launch_bounds__(256) void k_gemm_generic(int M, int N, int K, const int8_t *__restrict__ A,
@@ -876,28 +1094,103 @@ __global__ __launch_bounds__(256) void k_gemm_generic(int M, int N, int K, const
         }
 }
 
-template <int FM, int FN, int WM, int WN, bool ACC>
-hipError_t launch_mfma_acc(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C,
-                           hipStream_t s)
+// Tiles of k_gemm_tile.  T128 (one block per CU), T64 and T32x64 and T32 (several); the unaligned
+// form takes 64x128 tiles of eight 32x32 waves in place of T128 (its staging registers).
+enum Tile { T128, T64, T32x64, T32, NTILE };
+
+template <int WM, int WN, int FM, int FN, int KW, bool ALN>
+hipError_t launch_tile_as(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C, hipStream_t s, bool acc)
 {
-    constexpr int BM = WM * FM * 32, BN = WN * FN * 32;
+    constexpr int BM = WM * FM * 32, BN = WN * FN * 32, S = ALN ? 4 : 2;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    const bool edge = (M % BM) || (N % BN) || (K % BK);
-    if (edge)
-        hipLaunchKernelGGL((k_gemm_mfma<FM, FN, WM, WN, true, ACC>), dim3(tiles_m * tiles_n),
-                           dim3(WM * WN * 64), 0, s, M, N, K, A, B, C, tiles_m, tiles_n);
+    const dim3 grid(tiles_m * tiles_n), block(WM * WN * KW * 64);
+    if (acc)
+        hipLaunchKernelGGL((k_gemm_tile<WM, WN, FM, FN, KW, S, ALN, true>), grid, block, 0, s, M, N, K, A, B, C, tiles_m, tiles_n);
     else
-        hipLaunchKernelGGL((k_gemm_mfma<FM, FN, WM, WN, false, ACC>), dim3(tiles_m * tiles_n),
-                           dim3(WM * WN * 64), 0, s, M, N, K, A, B, C, tiles_m, tiles_n);
+        hipLaunchKernelGGL((k_gemm_tile<WM, WN, FM, FN, KW, S, ALN, false>), grid, block, 0, s, M, N, K, A, B, C, tiles_m, tiles_n);
     return hipGetLastError();
 }
-
-template <int FM, int FN, int WM, int WN>
-hipError_t launch_mfma(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C, hipStream_t s,
+hipError_t launch_tile(Tile t, bool aln, int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C, hipStream_t s,
                        bool acc)
 {
-    return acc ? launch_mfma_acc<FM, FN, WM, WN, true>(M, N, K, A, B, C, s)
-               : launch_mfma_acc<FM, FN, WM, WN, false>(M, N, K, A, B, C, s);
+    switch (t) {
+    case T128:
+        return aln ? launch_tile_as<4, 2, 1, 2, 1, true>(M, N, K, A, B, C, s, acc)
+                   : launch_tile_as<2, 4, 1, 1, 1, false>(M, N, K, A, B, C, s, acc);
+    case T64:
+        return aln ? launch_tile_as<2, 2, 1, 1, 2, true>(M, N, K, A, B, C, s, acc)
+                   : launch_tile_as<2, 2, 1, 1, 2, false>(M, N, K, A, B, C, s, acc);
+    case T32x64:
+        return aln ? launch_tile_as<1, 2, 1, 1, 2, true>(M, N, K, A, B, C, s, acc)
+                   : launch_tile_as<1, 2, 1, 1, 2, false>(M, N, K, A, B, C, s, acc);
+    default:
+        return aln ? launch_tile_as<1, 1, 1, 1, 4, true>(M, N, K, A, B, C, s, acc)
+                   : launch_tile_as<1, 1, 1, 1, 4, false>(M, N, K, A, B, C, s, acc);
+    }
+}
+
+// Estimated time (us) of a product on tile t: a start-up, C's traffic, and per 128-k stage the longer
+// of one block's own step (latency: few tiles) and the device's rate for all tiles (operand delivery
+// from L2, 12-16 TB/s: many tiles, which is why larger tiles win there).  Constants from graph
+// replays over M, N, K = 1 .. 4096 (us measured, T128 / T64 / T32x64 / T32, C = A.B):
+//   aligned   333x6144x2048  11.7 / 16.9 / 18.2 / 26.8    1024^3        7.7 / 5.6 / 6.2 / 8.3
+//             2048^3         15.0 / 23.6 / 29.8 / 47.3    17x4096x4096  15.1 / 7.1 / 6.4 / 6.6
+//             200x2048x2048   9.9 /  5.7 /  5.5 /  7.2    256^3         4.6 / 3.5 / 3.2 / 2.9
+//   unaligned 1001x1503x999  10.3 / 11.2 / 12.0 / 16.6    2047x300x2040 10.9 / 9.0 / 10.6 / 12.8
+//             33x2001x2001   13.5 / 10.1 /  8.3 /  7.3    37x41x257      5.4 / 4.3 / 4.1 / 3.6
+double c_us(int M, int N, bool acc) { return (double)M * N * (acc ? 8 : 4) / 6.5e6; }
+double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
+{
+    struct Cost {
+        int bm, bn;
+        double start, lat, thr;   // thr: a stage of 256 tiles
+    };
+    static const Cost costs[2][NTILE] = {
+        {{64, 128, 3.6, 0.60, 0.85}, {64, 64, 3.3, 0.38, 0.46}, {32, 64, 2.95, 0.33, 0.36}, {32, 32, 2.7, 0.25, 0.30}},
+        {{128, 128, 3.9, 0.35, 0.60}, {64, 64, 3.1, 0.12, 0.245}, {32, 64, 2.95, 0.10, 0.172}, {32, 32, 2.65, 0.095, 0.155}}};
+    const Cost &c = costs[aln][t];
+    const double tiles = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn), stages = (K + 127) / 128;
+    double per;
+    if (aln && t == T128) {   // one block per CU: whole rounds, and a last one that is at least a block's step
+        const double full = (double)((long)tiles / 256), rem = tiles - 256 * full;
+        per = full * c.thr + (rem > 0 ? fmax(c.lat, rem / 256 * c.thr) : 0.0);
+    } else {
+        per = fmax(c.lat, tiles / 256 * c.thr);
+    }
+    return c.start + c_us(M, N, acc) + per * stages;
+}
+Tile best_tile(bool aln, int M, int N, int K, bool acc, double &us)
+{
+    Tile best = T128;
+    us = tile_us(T128, aln, M, N, K, acc);
+    for (int t = T64; t < NTILE; t++) {
+        const double u = tile_us((Tile)t, aln, M, N, K, acc);
+        if (u < us) us = u, best = (Tile)t;
+    }
+    return best;
+}
+// k_gemm_big: rounds of 256 tiles, a last round no shorter than a block alone (4096^3 69.5 against 86
+// us on T128; 2048^2 x 4096, 64 tiles, 42 against 29).
+double big_us(int M, int N, int K, bool acc)
+{
+    const long tiles = (long)(M / 256) * (N / 256), full = tiles / 256, rem = tiles % 256;
+    return 3.0 + c_us(M, N, acc) + K / 128.0 * (full * 1.77 + (rem ? fmax(1.13, rem / 256.0 * 1.77) : 0.0));
+}
+// The split-K kernels for M <= 16 (C = A.B pays a clearing launch).  They stream B at up to 5 TB/s in
+// 128- or 256-column rows; the tiles reach 3.6 TB/s on a B beyond the caches, and less on rows that
+// are not whole cache lines (4x4112x4112: 7.0 us split-K, 9.4 on T32; 16x1280x1280: 7.7 and 3.7).
+double skinny_us(int M, int N, int K, bool acc)
+{
+    const double kn = (double)K * N, clear = acc ? 0.0 : 1.6;
+    if (N % 128 == 0 && K % 512 == 0) return clear + 2.9 + kn / 16e6;
+    return clear + (M <= 8 ? 4.7 + kn / 7e6 : 7.3 + kn / 4.3e6);
+}
+double skinny_tile_us(Tile &t, int M, int N, int K, bool acc)
+{
+    double us;
+    t = best_tile(true, M, N, K, acc, us);
+    if (N % 128) us = 2.65 + 1.5 * (us - 2.65);
+    return fmax(us, 2.65 + (double)K * N / 3.6e6);
 }
 
 // The 256x256 tile kernel k_gemm_big<NW, SUPER, ACC> (M, N multiples of 256, K % 64 == 0,
@@ -951,34 +1244,36 @@ hipError_t x100_gemm_i8_launch(int M, int N, int K, const int8_t *A, const int8_
 {
     const bool aligned = (K % 16 == 0) && (N % 16 == 0) && (((uintptr_t)A & 15) == 0) &&
                          (((uintptr_t)B & 15) == 0) && (((uintptr_t)C & 15) == 0);
+    // k_gemm_tile: 32-bit offsets inside a tile and a stage, and a whole 16-byte chunk in each operand
+    const bool tiled = N < (1 << 24) && K < (1 << 24) && (size_t)M * K >= 16 && (size_t)K * N >= 16;
+    const bool whole = M % 256 == 0 && N % 256 == 0 && K % BK == 0 && K >= 512;   // k_gemm_big
+    Tile tile = T128;
     if (variant == X100_GEMM_AUTO) {
-        if (!aligned)
-            variant = X100_GEMM_GENERIC;
-        else if (M <= 16 && (size_t)K * N < ((size_t)1 << 32))   // B must fit one buffer resource
+        double us = 0;
+        if (aligned && M <= 16 && (size_t)K * N < ((size_t)1 << 32) &&   // B must fit one buffer resource
+            (!tiled || skinny_us(M, N, K, acc) <= skinny_tile_us(tile, M, N, K, acc))) {
             variant = X100_GEMM_SKINNY;
-        // Tile by output size, measured at K = 1024-4096 (graph replay, us): 256x256 tiles from
-        // 4M outputs (2048^2 x 4096: 50.3 vs 52.6 with 128x128), 64x64 from 1M (1024^2 x 4096:
-        // 27.3 vs 39.9 / 45.2), 32x32 below (256^3: 3.5 vs 5.7; 512^3: 4.9 vs 7.9).  Smaller tiles
-        // put enough blocks on the 256 CUs when the product has few 256x256 tiles.
-        else if ((long)M * N >= 4L * 1024L * 1024L)
+        } else if (!tiled) {
+            variant = aligned && whole ? X100_GEMM_TILE256 : X100_GEMM_GENERIC;
+        } else {
+            tile = best_tile(aligned, M, N, K, acc, us);
+            if (!aligned || !whole || us < big_us(M, N, K, acc)) return launch_tile(tile, aligned, M, N, K, A, B, C, s, acc);
             variant = X100_GEMM_TILE256;
-        else if ((long)M * N >= 1024L * 1024L)
-            variant = X100_GEMM_TILE64;
-        else
-            variant = X100_GEMM_TILE32;
+        }
     }
     if (!aligned && variant != X100_GEMM_GENERIC) return hipErrorInvalidValue;
+    const bool tile_variant = variant == X100_GEMM_TILE128 || variant == X100_GEMM_TILE64 || variant == X100_GEMM_TILE32 ||
+                              ((variant == X100_GEMM_TILE256 || variant == X100_GEMM_TILE256_W4) && !whole);
+    if (tile_variant && !tiled) variant = X100_GEMM_GENERIC;
     switch (variant) {
     case X100_GEMM_TILE256:
-        // Full 256x256 tiles only; other shapes use the 128x128 tile with edge guards.
-        if (M % 256 || N % 256 || K % BK || K < 512) return launch_mfma<2, 2, 2, 2>(M, N, K, A, B, C, s, acc);
-        return launch_big<8>(M, N, K, A, B, C, s, acc);
+        // Full 256x256 tiles only; other shapes use the 128x128 tile.
+        return whole ? launch_big<8>(M, N, K, A, B, C, s, acc) : launch_tile(T128, true, M, N, K, A, B, C, s, acc);
     case X100_GEMM_TILE256_W4:
-        if (M % 256 || N % 256 || K % BK || K < 512) return launch_mfma<2, 2, 2, 2>(M, N, K, A, B, C, s, acc);
-        return launch_big<4>(M, N, K, A, B, C, s, acc);
-    case X100_GEMM_TILE128: return launch_mfma<2, 2, 2, 2>(M, N, K, A, B, C, s, acc);
-    case X100_GEMM_TILE64: return launch_mfma<1, 1, 2, 2>(M, N, K, A, B, C, s, acc);
-    case X100_GEMM_TILE32: return launch_mfma<1, 1, 1, 1>(M, N, K, A, B, C, s, acc);
+        return whole ? launch_big<4>(M, N, K, A, B, C, s, acc) : launch_tile(T128, true, M, N, K, A, B, C, s, acc);
+    case X100_GEMM_TILE128: return launch_tile(T128, true, M, N, K, A, B, C, s, acc);
+    case X100_GEMM_TILE64: return launch_tile(T64, true, M, N, K, A, B, C, s, acc);
+    case X100_GEMM_TILE32: return launch_tile(T32, true, M, N, K, A, B, C, s, acc);
     case X100_GEMM_SKINNY: {
         if (M > 16 || (size_t)K * N >= ((size_t)1 << 32)) return hipErrorInvalidValue;
         if (!acc) {

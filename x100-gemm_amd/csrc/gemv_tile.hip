@@ -7,7 +7,8 @@
 //   int4:  [N/8][K/32][128]  byte n*16 + k of tile (nb, kp) holds W[8nb + n][32kp + k] in the
 //                            low nibble and W[8nb + n][32kp + 16 + k] in the high nibble
 //                            (two's-complement 4-bit values).
-// One wave per 8-row N-block: lane l reads 16 bytes (row n = l % 8 of tile l / 8 of each 1 KiB
+// k_gemv_tile: dot products, for one or two token rows; k_gemv_tile_mm: the matrix cores (tile_mm says
+// which).  In k_gemv_tile one wave per 8-row N-block: lane l reads 16 bytes (row n = l % 8 of tile l / 8 of each 1 KiB
 // chunk), so a wave load is 64 x 16 contiguous bytes; all chunk loads of the wave are issued
 // before the first is used.  x rows sit in LDS with their 16-element sums.
 //
@@ -173,13 +174,103 @@ __global__ __launch_bounds__(256) void k_gemv_tile(int M, int N, int K, const ui
     }
 }
 
+// Several token rows on the matrix cores: v_mfma_i32_16x16x64_i8 with 16 weight rows (two N-blocks)
+// against the token rows as columns (columns from M on: copies, not stored).  A step is four 128-byte
+// tiles of each N-block, one 16-byte load per lane (lane l: row l % 8 of N-block l % 16 / 8, tile l / 16,
+// 512 contiguous bytes per N-block), which is one A operand (int8) or two (int4: the low nibbles
+// against the first 16 k of each tile, the high ones against the last 16, both as 16 q, so that the
+// sums are 16 times the result: |sum| <= 2^14 K, below 2^31 for every K that the LDS takes).  S waves
+// share the rows' steps.  x rows in LDS at a pitch of 16 mod 256 bytes: the 16 lanes of a read take 16
+// different 16-byte columns of a bank line.
+// U steps are loaded per pass, the first pass before x is waited for.  Bound by HBM on large matrices:
+// int4 151936 x 2048 at M = 8 54.7 -> 29.3 us (5.5 TB/s), where the dot products and the nibble
+// offsets of eight rows took longer than the weights.
+template <bool INT4, int S, int U>
+__global__ __launch_bounds__(256) void k_gemv_tile_mm(int M, int N, int K, int pitch, uint32_t mk16,
+                                                      const uint8_t *__restrict__ W, const int8_t *__restrict__ x,
+                                                      int32_t *__restrict__ y)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // x: [M][pitch] + a spare 16-byte slot
+    __shared__ v4i red[S > 1 ? 4 : 1][64];
+    const int lane = threadIdx.x & 63, w = wave_id(), g = lane >> 4, col = lane & 15;
+    const int Nb = N / 8, tiles = INT4 ? K / 32 : K / 16, steps = (tiles + 3) / 4;
+    const int rt = (int)blockIdx.x * (4 / S) + w / S, nb0 = 2 * rt;   // N-blocks nb0, nb0 + 1
+    const int sb = w % S * steps / S, se = (w % S + 1) * steps / S;
+    const rsrc_t wr = buf_rsrc(W + (size_t)min(nb0, Nb - 1) * tiles * 128, (uint32_t)(max(min(Nb - nb0, 2), 0) * tiles) * 128u);
+    const uint32_t off = (uint32_t)((col >> 3) * tiles * 128 + (col & 7) * 16);
+    auto load = [&](int s) __attribute__((always_inline)) {   // zeros past the steps, tiles or N-blocks
+        const int t = 4 * s + g;
+        return (v4i)__builtin_amdgcn_raw_buffer_load_b128(wr, (int)(s < se && t < tiles ? off + (uint32_t)t * 128u : ~0u), 0, 0);
+    };
+
+    const int vpr = K / 16, nv = M * vpr;
+    const rsrc_t xr = buf_rsrc(x, (uint32_t)M * K);
+    v4u xt[4];
+    xload(xr, 0, xt);
+    v4i wv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) wv[u] = load(sb + u);
+    __builtin_amdgcn_sched_barrier(0);
+    auto put = [&](int v0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int v = v0 + (int)threadIdx.x + 256 * i, r = (int)udiv16((uint32_t)min(v, nv), (uint32_t)vpr, mk16);
+            *(v4u *)(smem + (v < nv ? r * pitch + 16 * (v - r * vpr) : M * pitch)) = xt[i];
+        }
+    };
+    put(0);
+    for (int v0 = 1024; v0 < nv; v0 += 1024) {
+        xload(xr, v0, xt);
+        put(v0);
+    }
+    __syncthreads();
+
+    const uint8_t *xm = smem + min(col, M - 1) * pitch;
+    v4i acc0 = {}, acc1 = {};
+    for (int s0 = sb; s0 < se; s0 += U) {
+        if (s0 > sb) {
+#pragma unroll
+            for (int u = 0; u < U; u++) wv[u] = load(s0 + u);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int t = 4 * min(s0 + u, steps - 1) + g;   // past the last step: zero weights
+            if constexpr (INT4) {
+                v4i lo, hi;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    lo[j] = (wv[u][j] << 4) & (int)0xF0F0F0F0;
+                    hi[j] = wv[u][j] & (int)0xF0F0F0F0;
+                }
+                acc0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo, *(const v4i *)(xm + 32 * t), acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi, *(const v4i *)(xm + 32 * t + 16), acc1, 0, 0, 0);
+            } else {
+                v4i &a = u & 1 ? acc1 : acc0;
+                a = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[u], *(const v4i *)(xm + 16 * t), a, 0, 0, 0);
+            }
+        }
+    }
+    v4i v = acc0 + acc1;
+    if constexpr (S > 1) {
+        red[w][lane] = v;
+        __syncthreads();
+        if (w % S) return;
+#pragma unroll
+        for (int k = 1; k < S; k++) v += red[w + k][lane];
+    }
+    if constexpr (INT4) v >>= 4;
+    // rows 16 rt + 4 g + r of token row col
+    typedef int v4i_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    if (col < M && nb0 + (g >> 1) < Nb) *(v4i_a4 *)(y + (size_t)col * N + 16 * rt + 4 * g) = v;
+}
+
 // Waves per N-block: enough to give the chip ~1024 waves when the matrix has few N-blocks, as long
-// as every wave keeps at least 3 chunks (2 with several token rows, whose dot products dominate).
-inline int tile_split(int M, int N, int nch)
+// as every wave keeps at least 3 chunks.
+inline int tile_split(int N, int nch)
 {
     const int nblk = N / 8;
     const int by_waves = nblk >= 1024 ? 1 : nblk >= 512 ? 2 : 4;
-    const int minch = M >= 4 ? 2 : 3;
+    const int minch = 3;
     const int by_chunks = nch / 4 >= minch ? 4 : nch / 2 >= minch ? 2 : 1;
     return min(by_waves, by_chunks);
 }
@@ -200,11 +291,43 @@ template <int MR>
 hipError_t launch_tile(bool int4, int M, int N, int K, const void *W, const int8_t *x, int32_t *y, hipStream_t s)
 {
     const int tiles = int4 ? K / 32 : K / 16;
-    switch (tile_split(M, N, (tiles + 7) / 8)) {
+    switch (tile_split(N, (tiles + 7) / 8)) {
     case 1: return launch_tile_s<MR, 1>(int4, M, N, K, W, x, y, s);
     case 2: return launch_tile_s<MR, 2>(int4, M, N, K, W, x, y, s);
     default: return launch_tile_s<MR, 4>(int4, M, N, K, W, x, y, s);
     }
+}
+
+// k_gemv_tile_mm with S waves per 16 rows and U steps per pass (4 waves on K unless the rows alone fill
+// the chip and K is short; int8 from K = 1024 up with 8 steps in flight per wave).
+hipError_t launch_tile_mm(bool int4, int M, int N, int K, const void *W, const int8_t *x, int32_t *y, hipStream_t s)
+{
+    const int steps = ((int4 ? K / 32 : K / 16) + 3) / 4, pitch = (K + 255) / 256 * 256 + 16;
+    auto go = [&](auto k, int S) {
+        hipLaunchKernelGGL(k, dim3(((N / 8 + 1) / 2 * S + 3) / 4), dim3(256), (size_t)M * pitch + 16, s, M, N, K, pitch,
+                           udiv16_magic((uint32_t)(K / 16)), (const uint8_t *)W, x, y);
+    };
+    if (int4) {
+        if (N >= 16384 && steps <= 8) go(k_gemv_tile_mm<true, 2, 4>, 2);
+        else if (steps <= 8) go(k_gemv_tile_mm<true, 4, 2>, 4);
+        else go(k_gemv_tile_mm<true, 4, 4>, 4);
+    } else {
+        if (steps <= 8) go(k_gemv_tile_mm<false, 4, 2>, 4);
+        else if (steps <= 16) go(k_gemv_tile_mm<false, 4, 4>, 4);
+        else go(k_gemv_tile_mm<false, 4, 8>, 4);
+    }
+    return hipGetLastError();
+}
+
+// The matrix cores take several token rows; one row where the launch streams enough weights (us, dot
+// products / matrix cores; int4, int8): 151936x2048 M = 1 27.6 / 25.6, 47.5 / 44.5, M = 2 29.0 / 26.2,
+// M = 8 54.7 / 29.3, 60.6 / 48.3; 4864x896 M = 1 2.8 / 2.8, 3.2 / 3.2, M = 8 5.0 / 2.9, 5.3 / 3.2.  With
+// few rows and a long K, 2 or 3 rows stay on the dot products (256x4864 int8 M = 3 4.8 / 4.4, M = 2
+// 4.4 / 4.4; int4 3.6 / 3.7): too few 16-row tiles to split K over.
+inline bool tile_mm(bool int4, int M, int N, int K)
+{
+    if (M == 1) return N >= 65536 && K >= 1024;
+    return M > 2 || N >= 1024 || K <= 2048 || !int4;
 }
 
 }  // namespace
@@ -214,7 +337,7 @@ hipError_t x100_gemv_tile_launch(int int4, int M, int N, int K, const void *W, c
 {
     if (M < 1 || M > 8 || N < 8 || N % 8 || K < 16 || K % (int4 ? 32 : 16)) return hipErrorInvalidValue;
     if ((size_t)M * K + 16 + ((size_t)M * (K / 16) + 1) * 4 > 64 * 1024) return hipErrorInvalidValue;
+    if (tile_mm(int4 != 0, M, N, K)) return launch_tile_mm(int4 != 0, M, N, K, W, x, y, s);
     if (M == 1) return launch_tile<1>(int4 != 0, M, N, K, W, x, y, s);
-    if (M <= 4) return launch_tile<4>(int4 != 0, M, N, K, W, x, y, s);
-    return launch_tile<8>(int4 != 0, M, N, K, W, x, y, s);
+    return launch_tile<2>(int4 != 0, M, N, K, W, x, y, s);   // M = 2
 }

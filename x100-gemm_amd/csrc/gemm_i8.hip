@@ -14,8 +14,6 @@
 //   k_gemm_generic byte loads and scalar products: operands under 16 bytes, rows of 2^24 and more.
 #include <math.h>
 
-#include <type_traits>
-
 #include "x100_common.h"
 #include "x100_internal.h"
 
@@ -116,16 +114,6 @@ X100_DEV void store_c16(int32_t *dst, v4i v)
 {
     asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(v) : "memory");
 }
-
-// Calls f(std::integral_constant<int, i>) for i = 0 .. N-1 (indices usable as constants).
-template <int I, int N, class F> X100_DEV void static_for_impl(F &&f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for_impl<I + 1, N>(f);
-    }
-}
-template <int N, class F> X100_DEV void static_for(F &&f) { static_for_impl<0, N>(f); }
 
 template <int NW, int SUPER, bool ACC>
 __global__ __launch_bounds__(NW * 64) void k_gemm_big(int M, int N, int K, const int8_t *__restrict__ A,

@@ -7,8 +7,9 @@
 // qwen_moe_q3k.c:420-427), then every block's dot product is done in exact integer arithmetic
 // with v_dot4 and scaled in fp32.
 //
-// At M <= 8 the work is bandwidth bound: every lane issues all of its 16-byte weight loads before
-// it quantizes x, so a block's whole weight slice is in flight at once; no MFMA.
+// At M <= 8 the work is bandwidth bound: every lane issues its 16-byte weight loads before it
+// quantizes x.  With 5 to 8 rows of x the dot products take longer than the weights, and the 32-element
+// formats go to the matrix cores (k_q_mm; launch_mm says from where).
 //
 // Device weight layouts (made once at upload by x100q_pack):
 //   Q4_0  split into d[N*K/32] (fp16) and qs[N*K/32][16], so nibble rows are 16-byte aligned.
@@ -831,6 +832,219 @@ __global__ __launch_bounds__(NT) void k_q8_0(int M, int N, int K, int ngroups, c
     q8_0_body<MR, LPR, RPW, BPL, XPT, NT>(M, N, K, ngroups, wd, wq, x, y, blockIdx.x, gridDim.x);
 }
 
+// ------------------------------------------------------------------------------------------------
+// k_q_mm: Q4_0 and the int8 path for several token rows on the matrix cores.
+// Block = RT row tiles of 16 rows x KS waves; it quantizes x once into LDS and walks the tile groups
+// blockIdx.x, + gridDim.x, ...  v_mfma_i32_16x16x64_i8 takes 16 weight rows against 16 columns: columns
+// t and t + 8 are token t (columns of t >= M: copies, not stored) against different 32-element blocks
+// of the 64 k, the other block's x being zeros, so that every sum is one block's exact dot product and
+// both halves of the result are used:
+//   int8  lane l holds 16 bytes of row l % 16: blocks b, b + 1; one MFMA.
+//   Q4_0  lane l holds block b + l / 16 (nibbles as 16 (q - 8) in bytes): two MFMAs (low, high
+//         nibbles) for blocks b, b + 1 and two for b + 2, b + 3.
+// The scales and sums are those of k_q4_0 / k_q8_0 in their order, so the results have their bits:
+// LPR partial sums per row (partial j adds blocks j, j + LPR, ... in order), then a balanced tree over
+// j, which the DPP prefix sums of those kernels compute in their last lane.  Here the tree runs over
+// registers (a wave takes JN = LPR / KS consecutive j), columns t and t + 8, and the KS waves.
+// Weights are streamed from global memory straight into the operand registers (64 contiguous bytes per
+// row and load), CH loads ahead.  Bound by HBM on large matrices (151936 x 2048 int8: 5.0 TB/s) and by
+// the block's steps in turn (x's quantization, the scales, the products, the wave tree) on small ones.
+// ------------------------------------------------------------------------------------------------
+struct QmmLds {   // byte offsets; nbp = LPR * BPL blocks (zero scales from nb on)
+    int pitch, sx, zero, dw, red, total;
+};
+template <int JN, int BPL, int KS, int RT>
+__host__ __device__ constexpr QmmLds qmm_lds(int M)
+{
+    constexpr int nbp = JN * KS * BPL;
+    QmmLds l{};
+    l.pitch = 32 * nbp + 16;   // 16 mod 256 bytes: the tokens' reads fall on different LDS columns
+    l.sx = M * l.pitch;
+    l.zero = l.sx + nbp * 32;
+    l.dw = l.zero + 16;
+    l.red = l.dw + KS * RT * JN * BPL * 64;
+    l.total = l.red + (KS > 1 ? KS * RT * 512 : 0);
+    return l;
+}
+
+// FULL: K is exactly 32 LPR BPL (no range tests, divisions by constants).
+template <bool Q4, int JN, int BPL, int KS, int RT, int XPT, bool FULL>
+__global__ __launch_bounds__(64 * KS * RT) void k_q_mm(int M, int N, int K, int ngroups, uint32_t mnb, const uint16_t *__restrict__ wd,
+                                                   const uint8_t *__restrict__ wq, const float *__restrict__ x,
+                                                   float *__restrict__ y)
+{
+    constexpr int NT = 64 * KS * RT, LPR = JN * KS, JS = Q4 ? 4 : 2;   // j per step
+    constexpr int STEPS = JN / JS * BPL, CH = STEPS < 8 ? STEPS : 8, NCH = STEPS / CH;
+    constexpr int ND = JN * BPL / 4;                                   // scales per lane and tile
+    constexpr int BB = Q4 ? 16 : 32;                                   // bytes of a block's quants
+    static_assert(STEPS % CH == 0 && JN % JS == 0 && ND >= 1, "whole steps");
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const QmmLds L = qmm_lds<JN, BPL, KS, RT>(M);
+    const int nb = FULL ? LPR * BPL : K / 32;
+    const int lane = threadIdx.x & 63, w = wave_id(), ks = w % KS, g = lane >> 4, col = lane & 15, hf = col >> 3;
+    const int tok = min(col & 7, M - 1), j0 = ks * JN;
+    const uint32_t nblk = (uint32_t)N * (uint32_t)nb;   // < 2^27 (checked by the launcher)
+    const rsrc_t qr = buf_rsrc(wq, nblk * (uint32_t)BB), dr = buf_rsrc(wd, nblk * 2u);
+
+    // Step s = (j-step s / BPL, c = s % BPL): the lane's 16 bytes of row `row`; zeros past N or nb.
+    auto wload = [&](int row, auto sc) __attribute__((always_inline)) {
+        constexpr int s = decltype(sc)::value, jj = s / BPL, c = s % BPL;
+        const int b = j0 + JS * jj + LPR * c + (Q4 ? g : g >> 1);
+        const uint32_t blk = (row < N && (FULL || b < nb)) ? (uint32_t)row * (uint32_t)nb + (uint32_t)b : nblk;
+        return (v4i)__builtin_amdgcn_raw_buffer_load_b128(qr, (int)(blk * (uint32_t)BB + (Q4 ? 0u : 16u * (g & 1))), 0, 0);
+    };
+    // scale i of the lane: element e = 64 i + lane of [c][row][JN]
+    auto dload = [&](int row0, int i) __attribute__((always_inline)) {
+        const int e = 64 * i + lane, jl = e % JN, r = e / JN % 16, c = e / (16 * JN), b = j0 + jl + LPR * c;
+        const uint32_t blk = (row0 + r < N && (FULL || b < nb)) ? (uint32_t)(row0 + r) * (uint32_t)nb + (uint32_t)b : nblk;
+        return (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(dr, (int)(blk * 2u), 0, 0);
+    };
+    auto tile_row = [&](int gr) __attribute__((always_inline)) { return (gr * RT + w / KS) * 16; };
+
+    // x of the first pass, then the first tile's scales and weights, all in flight before x is used
+    const int total4 = M * nb * 8;
+    const rsrc_t xr = buf_rsrc(x, (uint32_t)total4 * 16u);
+    float4 xv[XPT];
+    x_load<XPT, NT>(xr, 0, xv);
+    int gr = blockIdx.x;
+    uint32_t dv[ND];
+    v4i wv[2][CH];
+    {
+        const int r0 = tile_row(gr);
+#pragma unroll
+        for (int i = 0; i < ND; i++) dv[i] = dload(r0, i);
+        static_for<CH>([&](auto u) __attribute__((always_inline)) { wv[0][decltype(u)::value] = wload(r0 + col, u); });
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // Quantize x: codes [token][pitch], scales [block][8 tokens]; the arithmetic of q8_0_from_regs.
+    float *sxp = (float *)(smem + L.sx);
+    for (int i = threadIdx.x; i < (LPR * BPL - nb) * 8; i += NT) sxp[nb * 8 + i] = 0.0f;
+    if (threadIdx.x < 4) ((int *)(smem + L.zero))[threadIdx.x] = 0;
+    for (int c0 = 0; c0 < total4; c0 += NT * XPT) {
+        if (c0 > 0) x_load<XPT, NT>(xr, c0, xv);
+#pragma unroll
+        for (int i = 0; i < XPT; i++) {
+            const int f = c0 + threadIdx.x + NT * i;
+            float d;
+            const uint32_t packed = q8_0_pack(xv[i], d);
+            if (f < total4) {
+                const int b = f >> 3, m = FULL ? b / nb : (int)udiv16((uint32_t)b, (uint32_t)nb, mnb), bl = b - m * nb;   // 32-blocks of the flattened rows
+                *(uint32_t *)(smem + m * L.pitch + 32 * bl + 4 * (f & 7)) = packed;
+                sxp[bl * 8 + m] = Q4 ? f16_trunc_pos(d) : d;   // the 8 lanes of a block hold the same d
+            }
+        }
+    }
+    __syncthreads();
+
+    // x operands: this lane's column takes block b + hf (set 0) or b + 2 + hf (set 1, Q4_0); lanes whose
+    // k belong to another block read the zeros.
+    const int kg = Q4 ? g : g >> 1;
+    const bool act0 = kg == hf, act1 = kg == 2 + hf;
+    const uint32_t xb = (uint32_t)(tok * L.pitch + 32 * (j0 + kg) + (Q4 ? 0 : 16 * (g & 1)));
+    const uint8_t *x0 = smem + (act0 ? xb : (uint32_t)L.zero), *x1 = smem + (act1 ? xb : (uint32_t)L.zero);
+    const int inc0 = act0 ? 1 : 0, inc1 = act1 ? 1 : 0, hi0 = act0 ? 16 : 0, hi1 = act1 ? 16 : 0;
+    const float *sxl = sxp + (j0 + hf) * 8 + tok;
+    float *dwl = (float *)(smem + L.dw) + w * (JN * BPL * 16);   // [c][JN][16 rows]
+    const float *dwr = dwl + hf * 16 + 4 * g;
+
+    for (; gr < ngroups; gr += gridDim.x) {
+        const int row0 = tile_row(gr), nrow0 = tile_row(gr + gridDim.x);
+        // this tile's scales to LDS (read by this wave only); the next tile's are requested
+#pragma unroll
+        for (int i = 0; i < ND; i++) {
+            const int e = 64 * i + lane, jl = e % JN, r = e / JN % 16, c = e / (16 * JN);
+            dwl[(c * JN + jl) * 16 + r] = h2f((uint16_t)dv[i]) * (Q4 ? 0.0625f : 1.0f);
+        }
+#pragma unroll
+        for (int i = 0; i < ND; i++) dv[i] = dload(nrow0, i);
+        v4f p[JN / 2];
+        static_for<NCH>([&](auto chc) __attribute__((always_inline)) {
+            constexpr int ch = decltype(chc)::value;
+            // the next chunk's weights, or the next tile's first
+            static_for<CH>([&](auto u) __attribute__((always_inline)) {
+                if constexpr (ch + 1 < NCH)
+                    wv[(ch + 1) & 1][decltype(u)::value] =
+                        wload(row0 + col, std::integral_constant<int, (ch + 1) * CH + decltype(u)::value>{});
+                else
+                    wv[(ch + 1) & 1][decltype(u)::value] = wload(nrow0 + col, u);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<CH>([&](auto uc) __attribute__((always_inline)) {
+                constexpr int u = decltype(uc)::value, s = ch * CH + u, jj = s / BPL, c = s % BPL, bo = JS * jj + LPR * c;
+                const v4i q = wv[ch & 1][u];
+                constexpr int set = Q4 ? 2 : 1;
+#pragma unroll
+                for (int t = 0; t < set; t++) {
+                    const uint8_t *xp = (t ? x1 : x0) + 32 * bo * (t ? inc1 : inc0);
+                    v4i D;
+                    if constexpr (Q4) {
+                        const v4u qu = (v4u)q;
+                        const v4i lo = (v4i)(((qu << 4) & 0xF0F0F0F0u) ^ 0x80808080u), hi = (v4i)((qu & 0xF0F0F0F0u) ^ 0x80808080u);
+                        D = __builtin_amdgcn_mfma_i32_16x16x64_i8(lo, *(const v4i *)xp, v4i{0, 0, 0, 0}, 0, 0, 0);
+                        D = __builtin_amdgcn_mfma_i32_16x16x64_i8(hi, *(const v4i *)(xp + (t ? hi1 : hi0)), D, 0, 0, 0);
+                    } else {
+                        D = __builtin_amdgcn_mfma_i32_16x16x64_i8(q, *(const v4i *)xp, v4i{0, 0, 0, 0}, 0, 0, 0);
+                    }
+                    const float sx = sxl[8 * (bo + 2 * t)];
+                    const v4f dw = *(const v4f *)(dwr + ((JS * jj + 2 * t) + c * JN) * 16);
+                    v4f &a = p[jj * (JS / 2) + t];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float ds = dw[r] * sx;
+                        if constexpr (Q4) {
+                            const float term = (float)D[r] * ds;
+                            a[r] = (c == 0 ? 0.0f : a[r]) + term;
+                        } else {
+                            a[r] = __builtin_fmaf(ds, (float)D[r], c == 0 ? 0.0f : a[r]);
+                        }
+                    }
+                    if constexpr (c == BPL - 1)   // partials j and j + 1: columns t and t + 8
+#pragma unroll
+                        for (int r = 0; r < 4; r++) a[r] += dpp_f<0x128>(0.0f, a[r]);
+                }
+            });
+        });
+        if constexpr (NCH & 1) {
+#pragma unroll
+            for (int u = 0; u < CH; u++) wv[0][u] = wv[1][u];
+        }
+#pragma unroll
+        for (int n = JN / 4; n >= 1; n /= 2)
+#pragma unroll
+            for (int i = 0; i < n; i++) p[i] = p[2 * i] + p[2 * i + 1];
+        typedef float v4f_a4 __attribute__((ext_vector_type(4), aligned(4)));
+        v4f v = p[0];
+        if constexpr (KS > 1) {
+            v4f *red = (v4f *)(smem + L.red);   // [RT][KS][4 g][8 tokens]
+            if (col < 8) red[w * 32 + g * 8 + col] = v;
+            __syncthreads();
+            if (ks == 0) {
+                v4f s[KS];
+#pragma unroll
+                for (int k = 0; k < KS; k++) s[k] = red[(w + k) * 32 + g * 8 + (col & 7)];
+#pragma unroll
+                for (int n = KS / 2; n >= 1; n /= 2)
+#pragma unroll
+                    for (int i = 0; i < n; i++) s[i] = s[2 * i] + s[2 * i + 1];
+                v = s[0];
+            }
+        }
+        if (ks == 0 && col < M) {   // col < 8: M <= 8
+            const int r0 = row0 + 4 * g;
+            float *yp = y + (size_t)col * N + r0;
+            if (r0 + 4 <= N) {
+                *(v4f_a4 *)yp = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (r0 + r < N) yp[r] = v[r];
+            }
+        }
+        if constexpr (KS > 1) __syncthreads();   // red is read before the next tile writes it
+    }
+}
+
 // A decoder layer's q, v and k projections in one launch: blocks 0 .. nb0-1 compute a0 and
 // nb0 .. nb01-1 a1 (one-row K-quant products, as k_kq_rm2), the rest the int8-path product of
 // one token row with the plan of k_q8_0<1, 16, 1, 4, 2, 256> (33 to 64 blocks of 32 per row); each
@@ -1162,6 +1376,59 @@ hipError_t launch_q8_0(int M, int N, int K, const void *w, const float *x, float
     return launch_q8_0_x<MR, 64, 8>(M, N, K, w, x, y, s);
 }
 
+// k_q_mm plans.  The grid is the blocks resident at once, or one per tile group if there are fewer.
+template <bool Q4, int JN, int BPL, int KS, int RT, int XPT>
+hipError_t launch_q_mm(int M, int N, int K, const void *w, const float *x, float *y, hipStream_t s)
+{
+    constexpr int NT = 64 * KS * RT;
+    const int nb = K / 32, lds = qmm_lds<JN, BPL, KS, RT>(M).total, groups = (N + 16 * RT - 1) / (16 * RT);
+    const size_t ngrp = (size_t)N * nb;
+    const uint16_t *wd = (const uint16_t *)w;
+    const uint8_t *wq = (const uint8_t *)w + align256(ngrp * 2);
+    auto go = [&](auto k) {
+        const int res = resident_blocks(k, NT, lds);
+        hipLaunchKernelGGL(k, dim3(groups < res ? groups : res), dim3(NT), lds, s, M, N, K, groups,
+                           udiv16_magic((uint32_t)nb), wd, wq, x, y);
+    };
+    if (nb == JN * KS * BPL) go(k_q_mm<Q4, JN, BPL, KS, RT, XPT, true>);
+    else go(k_q_mm<Q4, JN, BPL, KS, RT, XPT, false>);
+    return hipGetLastError();
+}
+// Where the matrix cores win (us, k_q_mm against the dot-product kernels, M = 8 unless said; LPR and BPL
+// as those kernels take them from K).  The plans spread x's quantization over 512 or 1024 threads;
+// with few rows of x the dot products cost less than that spread's fixed steps.
+//   int8  K <= 512, M >= 2 (777x480: M = 2 2.7 / 3.2, M = 8 2.9 / 5.2)
+//         K <= 1024, M >= 3 (4096x1024: M = 3 3.5 / 3.8, M = 8 3.8 / 5.4)
+//         K <= 4096, M >= 5 (4096x2048 5.1 / 6.7, M = 4 4.6 / 4.5; 151936x2048 68 / 80, M = 4 65 / 61;
+//                            8192x4096 11.8 / 15.8)
+//         K <= 8192, M >= 7 (4099x8000 16.8 / 20.2, 2048x8192 14.3 / 14.6, M = 5 13.1 / 11.8)
+//   Q4_0  M >= 5 (4096x4096 7.8 / 11.2, 32768x4096 20 / 50), or many rows (16384x2048: M = 2 7.7 / 8.7;
+//         9000x4096: M = 3 10.2 / 10.9, M = 2 9.9 / 9.2; 32768x4096: M = 2 18.6 / 21.5), or K > 4096
+//         (3000x7680: M = 2 8.9 / 9.2, M = 4 10.0 / 11.9)
+// hipErrorNotSupported: outside (the caller takes those kernels).
+hipError_t launch_mm(bool q4, int M, int N, int K, const void *w, const float *x, float *y, hipStream_t s)
+{
+    const int nb = K / 32;
+    if (M < 2 || nb > 256 || (size_t)N * nb >= ((size_t)1 << 27)) return hipErrorNotSupported;
+    if (q4) {
+        if (nb > 128) return launch_q_mm<true, 4, 4, 16, 1, 8>(M, N, K, w, x, y, s);
+        if (M < 5 && N < (M == 2 && nb > 64 ? 16384 : 8192)) return hipErrorNotSupported;
+        if (nb > 64)
+            return N >= 16384 ? launch_q_mm<true, 8, 2, 8, 2, 8>(M, N, K, w, x, y, s)
+                              : launch_q_mm<true, 4, 2, 16, 1, 8>(M, N, K, w, x, y, s);
+        return N >= 4096 ? launch_q_mm<true, 8, 1, 8, 2, 4>(M, N, K, w, x, y, s)
+                         : launch_q_mm<true, 4, 1, 16, 1, 4>(M, N, K, w, x, y, s);
+    }
+    if (nb <= 16) return launch_q_mm<false, 4, 1, 4, 1, 4>(M, N, K, w, x, y, s);
+    if (nb <= 32) return M >= 3 ? launch_q_mm<false, 4, 2, 4, 1, 8>(M, N, K, w, x, y, s) : hipErrorNotSupported;
+    if (M < (nb <= 128 ? 5 : 7)) return hipErrorNotSupported;
+    if (nb <= 64)
+        return N >= 8192 ? launch_q_mm<false, 2, 4, 8, 2, 4>(M, N, K, w, x, y, s)
+                         : launch_q_mm<false, 2, 4, 8, 1, 8>(M, N, K, w, x, y, s);
+    return nb <= 128 ? launch_q_mm<false, 2, 4, 16, 1, 8>(M, N, K, w, x, y, s)
+                     : launch_q_mm<false, 4, 4, 16, 1, 8>(M, N, K, w, x, y, s);
+}
+
 // K-quant launch plan: RB = ceil(N / 256) rows per block (about one block per CU), at most 256 / nsb
 // (so at most 16 waves of 16 four-lane units); nw = the waves of the two-lane row-major kernel;
 // false when the block's LDS would exceed 160 KiB.
@@ -1347,6 +1614,10 @@ hipError_t x100_qgemv_launch(int qtype, int M, int N, int K, const void *w, cons
                              hipStream_t s)
 {
     if (!x100_qgemv_supported(qtype, M, N, K)) return hipErrorInvalidValue;
+    if (qtype != X100_Q4_K && qtype != X100_Q3_K) {
+        const hipError_t e = launch_mm(qtype == X100_Q4_0, M, N, K, w, x, y, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     if (qtype == X100_Q4_0) {
         if (M == 1) return launch_q4_0<1>(M, N, K, w, x, y, s);
         if (M <= 4) return launch_q4_0<4>(M, N, K, w, x, y, s);

@@ -9,11 +9,24 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 #define X100_DEV __device__ __forceinline__
+
+// Calls f(std::integral_constant<int, i>) for i = 0 .. N-1 (indices usable as constants).
+template <int I, int N, class F> X100_DEV void static_for_impl(F &&f)
+{
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for_impl<I + 1, N>(f);
+    }
+}
+template <int N, class F> X100_DEV void static_for(F &&f) { static_for_impl<0, N>(f); }
 
 // GGUF type ids (bench/gguf_dump.c:12-13 of the reference).
 enum { X100_Q4_0 = 2, X100_Q8_0 = 8, X100_Q3_K = 11, X100_Q4_K = 12, X100_Q5_K = 13, X100_Q6_K = 14 };
@@ -320,23 +333,29 @@ X100_DEV float f16_trunc_pos(float d)
     const float r = d >= 0x1p-14f ? nrm : sub;
     return d >= 65536.0f ? __builtin_inff() : r;
 }
+// The lane's four codes of a 32-element block held by 8 consecutive lanes, and the block's fp32 scale.
+X100_DEV uint32_t q8_0_pack(const float4 v, float &d)
+{
+    constexpr float RND = 0x1.8p23f;
+    const float a = max8_f(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    const float amax = fmaxf(a, 1e-6f);
+    d = div127_rn(amax);
+    const float inv = rcp_rn(d);
+    const float p0 = v.x * inv, p1 = v.y * inv, p2 = v.z * inv, p3 = v.w * inv;
+    const uint32_t t0 = __float_as_uint(p0 + RND), t1 = __float_as_uint(p1 + RND);
+    const uint32_t t2 = __float_as_uint(p2 + RND), t3 = __float_as_uint(p3 + RND);
+    return perm(t1, t0, 0x0c0c0400u) | perm(t3, t2, 0x04000c0cu);
+}
 template <int XPT, int NT = 256, bool F16D = true, bool OFS = true>
 X100_DEV void q8_0_from_regs(const float4 (&v)[XPT], int c0, int total4, int K, int8_t *xlo,
                              int8_t *xhi, float *xd, int *xs)
 {
     (void)K;   // rows are contiguous and K % 32 == 0: element e is in 32-block e / 32
-    constexpr float RND = 0x1.8p23f;
 #pragma unroll
     for (int i = 0; i < XPT; i++) {
         const int f = c0 + threadIdx.x + NT * i;
-        const float a = max8_f(fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
-        const float amax = fmaxf(a, 1e-6f);
-        const float d = div127_rn(amax);
-        const float inv = rcp_rn(d);
-        const float p0 = v[i].x * inv, p1 = v[i].y * inv, p2 = v[i].z * inv, p3 = v[i].w * inv;
-        const uint32_t t0 = __float_as_uint(p0 + RND), t1 = __float_as_uint(p1 + RND);
-        const uint32_t t2 = __float_as_uint(p2 + RND), t3 = __float_as_uint(p3 + RND);
-        const uint32_t packed = perm(t1, t0, 0x0c0c0400u) | perm(t3, t2, 0x04000c0cu);
+        float d;
+        const uint32_t packed = q8_0_pack(v[i], d);
         const int pos = 4 * (f & 7);
         const int b = f < total4 ? f >> 3 : total4 >> 3;   // spare block past the end
         int8_t *dst = pos < 16 ? xlo + b * 16 + pos : xhi + b * 16 + (pos - 16);

@@ -859,9 +859,12 @@ __global__ __launch_bounds__(256) void k_moe_act_q8k(int P, int ff, MoeWs ws)
 //   A = the pairs' Q8_K bytes of sub-block j (lane l: pair l % 32, elements 16 * (l / 32) .. +16),
 //   B = the weight rows' 4-bit values of sub-block j times the low or the high 3 bits of the
 //       row's 6-bit scale (lane l: row l % 32, the same elements),
-// so the two accumulators hold sum_j sc_lo_j dot_j and sum_j sc_hi_j dot_j exactly; a third
-// chain whose B holds m_j in every byte gives the min term sum_j m_j * (sum of the activation
-// bytes of sub-block j).  These integers equal those of the one-row kernels, and the fp32 combine
+// so the two accumulators hold sum_j sc_lo_j dot_j and sum_j sc_hi_j dot_j exactly.  The min term
+// sum_j m_j S_j (S_j the sum of the activation bytes of sub-block j, S_j = l_j + 64 h_j) takes two
+// v_mfma_i32_32x32x16_i8 per super-block, the m_j against the bytes l_j and h_j that the block packs
+// into LDS once: in place of one full product per sub-block with m_j in every byte (a quarter of the
+// matrix work, and four register copies of each m_j).  Bound by the VALU, whose unpacking and scaling
+// fill it 70% (M = 512).  These integers equal those of the one-row kernels, and the fp32 combine
 // per super-block (q4k_combine) and the sum over super-blocks run in the same order, so every
 // output is bit-identical to theirs.
 //
@@ -878,6 +881,9 @@ constexpr int MF_PCH = 32;   // pairs per chunk of the MFMA path
 // staging round trip; the down projection of ff = 768 has 3), else the first half rounded up to
 // even, so that the halves meet between two ring steps.
 __host__ __device__ inline int mf_half(int nsb) { return nsb <= 4 ? nsb : min(nsb, ((nsb + 1) / 2 + 1) & ~1); }
+
+// Dynamic LDS: the staged activations, then the sums per sub-block.
+inline size_t mf_lds(int nsb) { return (size_t)mf_half(nsb) * 8192 + (size_t)nsb * 512; }
 
 template <bool GU, bool TL, int RT>
 __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, const uint8_t *__restrict__ Wa,
@@ -942,6 +948,24 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
     // DMA lane l fetches pair l % 32, bytes 16 * (l / 32) .. +16 of each sub-block.
     const uint8_t *src = X + (size_t)arow * rec + 16 * h;
     const int nh1 = mf_half(nsb);   // nsb, or even: the halves meet between two ring steps
+    // the sums per sub-block of pair t % 32: bytes {l_0..3, h_0..3, l_4..7, h_4..7} at [super-block][pair]
+    uint8_t *s_bs = smem + nh1 * 8192;
+    for (int sb = t >> 5; sb < nsb; sb += 8) {
+        const v4i *bp = (const v4i *)(X + (size_t)arow * rec + nsb * 256 + sb * 64);
+        v4i o;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const v4i b0 = bp[2 * k], b1 = bp[2 * k + 1];
+            const int s0 = b0[0] + b0[1], s1 = b0[2] + b0[3], s2 = b1[0] + b1[1], s3 = b1[2] + b1[3];
+            const uint32_t w01 = perm((uint32_t)s1, (uint32_t)s0, 0x05040100u) , w23 = perm((uint32_t)s3, (uint32_t)s2, 0x05040100u);
+            // 16-bit sums, two per dword: their low 6 bits, and the rest as signed bytes
+            const uint32_t l01 = w01 & 0x003f003fu, l23 = w23 & 0x003f003fu;
+            const uint32_t h01 = (w01 >> 6) & 0x00ff00ffu, h23 = (w23 >> 6) & 0x00ff00ffu;
+            o[2 * k] = (int)perm(l23, l01, 0x06040200u);
+            o[2 * k + 1] = (int)perm(h23, h01, 0x06040200u);
+        }
+        *(v4i *)(s_bs + (sb * 32 + col) * 16) = o;
+    }
     auto stage = [&](int sb0, int sb1) {
         for (int c = 8 * sb0 + w; c < 8 * sb1; c += 4) dma_1k(src + 32 * c, smem + (c - 8 * sb0) * 1024);
     };
@@ -963,22 +987,25 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
     // 16-bit multiply per dword scales four bytes at once (each byte product stays below 256).
     auto compute = [&](int sb, const Wt &o) {
         const uint8_t *as = smem + (sb < nh1 ? sb : sb - nh1) * 8 * 1024 + lane * 16;
-        int sc[8], mm[8];
-        v16i lo = {}, hi = {}, imn = {};
+        v16i lo = {}, hi = {};
         v4i a[9];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            int m;
-            gsm(o.hdr, j, sc[j], m);
-            mm[j] = (int)__builtin_amdgcn_perm((uint32_t)m, (uint32_t)m, 0u);   // m in every byte
-        }
+        // get_scale_min_k4 of the eight sub-blocks, four bytes at a time; the 3-bit halves of the scales
+        const uint32_t d1 = (uint32_t)o.hdr[1], d2 = (uint32_t)o.hdr[2], d3 = (uint32_t)o.hdr[3];
+        const uint32_t sc[2] = {d1 & 0x3F3F3F3Fu, (d3 & 0x0F0F0F0Fu) | ((d1 >> 2) & 0x30303030u)};
+        const uint32_t mn = h ? ((d3 >> 4) & 0x0F0F0F0Fu) | ((d2 >> 2) & 0x30303030u) : d2 & 0x3F3F3F3Fu;   // m_4h .. +3
+        const uint32_t s_lo[2] = {sc[0] & 0x07070707u, sc[1] & 0x07070707u};
+        const uint32_t s_hi[2] = {(sc[0] >> 3) & 0x07070707u, (sc[1] >> 3) & 0x07070707u};
+        const uint64_t bs = *(const uint64_t *)(s_bs + (sb * 32 + col) * 16 + 8 * h);   // l | h of sub-blocks 4h ..
         a[0] = *(const v4i *)as;
+        const v16i ml = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)bs, (long)(uint64_t)mn, v16i{}, 0, 0, 0);
+        const v16i mh = __builtin_amdgcn_mfma_i32_32x32x16_i8((long)bs, (long)((uint64_t)mn << 32), v16i{}, 0, 0, 0);
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             if (j < 7) a[j + 1] = *(const v4i *)(as + (j + 1) * 1024);
             const v4i b = (o.q[j >> 1] >> (4 * (j & 1))) & 0x0F0F0F0F;
-            const u16x2 slo = u16x2{(uint16_t)(sc[j] & 7), (uint16_t)(sc[j] & 7)};
-            const u16x2 shi = u16x2{(uint16_t)(sc[j] >> 3), (uint16_t)(sc[j] >> 3)};
+            const uint32_t sel = 0x0c000c00u | (uint32_t)(j & 3) * 0x00010001u;   // byte j % 4 in both halves
+            const u16x2 slo = __builtin_bit_cast(u16x2, perm(0u, s_lo[j >> 2], sel));
+            const u16x2 shi = __builtin_bit_cast(u16x2, perm(0u, s_hi[j >> 2], sel));
             v4i blo, bhi;
 #pragma unroll
             for (int t = 0; t < 4; t++) {
@@ -990,7 +1017,6 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
             }
             lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[j], blo, lo, 0, 0, 0);
             hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[j], bhi, hi, 0, 0, 0);
-            imn = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[j], v4i{mm[j], mm[j], mm[j], mm[j]}, imn, 0, 0, 0);
         }
 #pragma unroll
         for (int qd = 0; qd < 4; qd++)
@@ -998,7 +1024,7 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
 #pragma unroll
                 for (int r = 4 * qd; r < 4 * qd + 4; r++) {
                     const int k = 8 * (r >> 2) + 4 * h + (r & 3);   // chunk pair of accumulator register r
-                    acc[r] = acc[r] + q4k_combine(o.hdr, s_dx[sb][k], lo[r] + 8 * hi[r], imn[r]);
+                    acc[r] = acc[r] + q4k_combine(o.hdr, s_dx[sb][k], lo[r] + 8 * hi[r], ml[r] + 64 * mh[r]);
                 }
     };
     const int nstep = RT * nsb;
@@ -1390,15 +1416,15 @@ hipError_t moe_launch_mfma(int M, int d, int ff, int n_exp, int n_act, const flo
     route_rows(M, d, n_exp, hn, R, ws, s);
     hipLaunchKernelGGL(k_moe_topk_rows, dim3(nrc), dim3(512), 0, s, M, n_exp, n_act, ws, sel, sw);
     hipLaunchKernelGGL(k_moe_group<MF_PCH>, dim3(1), dim3(256), 0, s, P, n_exp, ws);
-    hipLaunchKernelGGL((k_moe_mfma<true, TL, 1>), dim3(Vmax, ff / 64), dim3(256), (size_t)mf_half(nsb) * 8192, s, d,
+    hipLaunchKernelGGL((k_moe_mfma<true, TL, 1>), dim3(Vmax, ff / 64), dim3(256), mf_lds(nsb), s, d,
                        ff, n_act, (const uint8_t *)Wg, (const uint8_t *)Wu, ws);
     hipLaunchKernelGGL(k_moe_act_q8k, dim3((P * nsf + 3) / 4), dim3(256), 0, s, P, ff, ws);
     // down: MF_DN_RT row tiles per wave when one staging part holds every super-block
     if (MF_DN_RT > 1 && mf_half(nsf) == nsf && d % (128 * MF_DN_RT) == 0)
         hipLaunchKernelGGL((k_moe_mfma<false, TL, MF_DN_RT>), dim3(Vmax, d / (128 * MF_DN_RT)), dim3(256),
-                           (size_t)nsf * 8192, s, d, ff, n_act, (const uint8_t *)Wd, (const uint8_t *)nullptr, ws);
+                           mf_lds(nsf), s, d, ff, n_act, (const uint8_t *)Wd, (const uint8_t *)nullptr, ws);
     else
-        hipLaunchKernelGGL((k_moe_mfma<false, TL, 1>), dim3(Vmax, d / 128), dim3(256), (size_t)mf_half(nsf) * 8192, s, d,
+        hipLaunchKernelGGL((k_moe_mfma<false, TL, 1>), dim3(Vmax, d / 128), dim3(256), mf_lds(nsf), s, d,
                            ff, n_act, (const uint8_t *)Wd, (const uint8_t *)nullptr, ws);
     hipLaunchKernelGGL(k_moe_combine, dim3((M * d + 255) / 256), dim3(256), 0, s, M, d, n_act, ws, out, residual,
                        (const float *)nullptr);

@@ -404,6 +404,69 @@ __global__ __launch_bounds__(256) void k_moe_route_rows(int M, int d, int n_exp,
     }
 }
 
+// The same for d <= 2048 from LDS: a block of 4 waves stages its eb experts' router rows once for 4 * RR_ROWS token rows, RR_ROWS in each wave's registers, so that no
+// wave waits for memory between its dots.  EXACT: d = 2048 (no range tests).
+// grid (ceil(n_exp / eb) + ceil(4 * RR_ROWS * d / 1024), ceil(M / (4 * RR_ROWS))).
+template <bool EXACT>
+__global__ __launch_bounds__(256) void k_moe_route_tile(int M, int d, int n_exp, int eb, const float *__restrict__ hn,
+                                                        const float *__restrict__ R, MoeWs ws)
+{
+    constexpr int NJ = 8;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [eb][d] floats
+    const int lane = threadIdx.x & 63, w = wave_id();
+    const int nsb = EXACT ? NJ : d / 256;
+    const int row0 = blockIdx.y * 4 * RR_ROWS, nr = min(4 * RR_ROWS, M - row0);
+    const int ngrp = (n_exp + eb - 1) / eb;
+    if ((int)blockIdx.x >= ngrp) {   // quantizer blocks: one wave per 256-element block of the rows
+        const int q = ((int)blockIdx.x - ngrp) * 4 + w;
+        if (q >= nr * nsb) return;
+        const int m = q / nsb, sb = q - m * nsb;
+        const float4 v = *(const float4 *)(hn + (size_t)(row0 + m) * d + sb * 256 + 4 * lane);
+        uint8_t *rec = ws.xrec + (size_t)(row0 + m) * q8k_rec_bytes(nsb);
+        q8_K_wave(v, (int8_t *)rec + sb * 256, (int *)(rec + nsb * 256) + sb * 16, (float *)(rec + nsb * 320) + sb);
+        return;
+    }
+    const int e0 = blockIdx.x * eb, ne = min(eb, n_exp - e0);
+    const int mb = w * RR_ROWS;   // the wave's rows row0 + mb ..
+    float4 hv[RR_ROWS][NJ];
+#pragma unroll
+    for (int m = 0; m < RR_ROWS; m++) {
+        const rsrc_t hr = buf_rsrc(hn + (size_t)(row0 + min(mb + m, nr - 1)) * d, (uint32_t)d * 4u);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) hv[m][j] = buf_load_f4(hr, (uint32_t)(4 * lane + 256 * j) * 4u);
+    }
+    for (int ch = w; ch < ne * nsb; ch += 4)   // the experts' rows are contiguous: 1 KiB copies
+        dma_1k(R + (size_t)e0 * d + (size_t)ch * 256 + 4 * lane, smem + ch * 1024);
+    __syncthreads();
+    if (mb >= nr) return;
+    for (int i = 0; i < ne; i++) {
+        const float4 *rp = (const float4 *)smem + (size_t)i * nsb * 64 + lane;
+        float4 rv[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; j++) rv[j] = rp[64 * (EXACT ? j : min(j, nsb - 1))];
+        float sum[RR_ROWS];   // each row's sum in k_moe_route's order (blocks j ascending, then x, y, z, w)
+#pragma unroll
+        for (int m = 0; m < RR_ROWS; m++) sum[m] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            if (EXACT || j < nsb) {
+#pragma unroll
+                for (int m = 0; m < RR_ROWS; m++) sum[m] += rv[j].x * hv[m][j].x;
+#pragma unroll
+                for (int m = 0; m < RR_ROWS; m++) sum[m] += rv[j].y * hv[m][j].y;
+#pragma unroll
+                for (int m = 0; m < RR_ROWS; m++) sum[m] += rv[j].z * hv[m][j].z;
+#pragma unroll
+                for (int m = 0; m < RR_ROWS; m++) sum[m] += rv[j].w * hv[m][j].w;
+            }
+#pragma unroll
+        for (int m = 0; m < RR_ROWS; m++) sum[m] = wave_sum_bfly_f(sum[m]);
+#pragma unroll
+        for (int m = 0; m < RR_ROWS; m++)
+            if (lane == 0 && mb + m < nr) ws.logits[(size_t)(row0 + mb + m) * n_exp + e0 + i] = sum[m];
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // Routing of all M rows from the logits, computed identically by every gate/up block.
 // Softmax over all experts (max-subtract, exp, times 1/sum; lane l of a wave holds experts
@@ -1393,6 +1456,20 @@ MoeWs carve(uintptr_t base, int M, int d, int ff, int n_exp, int n_act, size_t *
 
 void route_rows(int M, int d, int n_exp, const float *hn, const float *R, MoeWs ws, hipStream_t s)
 {
+    // From 48 rows at d <= 2048 the LDS form, with the experts per block that leave 512 blocks or more, at
+    // most 4 (us, k_moe_route_rows / 1, 2, 4, 8 experts; 128 experts, d = 2048: M = 512 21.7 / 24.6, 18.9,
+    // 17.4, 20.0; M = 256 14.6 / 13.5, 11.2, 9.9, 12.6; M = 128 7.9 / 8.4, 5.9, 7.7, 9.3; M = 64 5.6 / 5.6,
+    // 5.4; M = 17 3.5 / 4.4; 512 rows, 60 experts, d = 1536 23.3 / 13.3, 10.9, 10.2).
+    if (d <= 2048 && M >= 48) {
+        const int rg = (M + 4 * RR_ROWS - 1) / (4 * RR_ROWS), eb = max(1, min(4, rg * n_exp / 512));
+        const dim3 g((n_exp + eb - 1) / eb + (4 * RR_ROWS * (d / 256) + 3) / 4, rg);
+        const size_t lds = (size_t)eb * d * 4;
+        if (d == 2048)
+            hipLaunchKernelGGL(k_moe_route_tile<true>, g, dim3(256), lds, s, M, d, n_exp, eb, hn, R, ws);
+        else
+            hipLaunchKernelGGL(k_moe_route_tile<false>, g, dim3(256), lds, s, M, d, n_exp, eb, hn, R, ws);
+        return;
+    }
     const int epw = max(1, min(8, M / 64));   // experts per wave
     const int ngrp = (n_exp + 4 * epw - 1) / (4 * epw), nq = (RR_ROWS * (d / 256) + 3) / 4;
     const dim3 g(ngrp + nq, (M + RR_ROWS - 1) / RR_ROWS);

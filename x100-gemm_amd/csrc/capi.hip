@@ -153,8 +153,9 @@ bool moe_ptrs_ok(const float *hn, const float *R, const void *Wg, const void *Wu
     return !(((uintptr_t)hn | (uintptr_t)R | (uintptr_t)Wg | (uintptr_t)Wu | (uintptr_t)Wd) & 15);
 }
 
-// Host copies of the host-pointer GEMM: one range split in nt equal parts, copied by the caller and
-// nt - 1 worker threads (a pageable <-> pinned copy runs at 29 GB/s on one core, 76-80 GB/s on 4-8).
+// Host copies and int32 additions of the host-pointer GEMM: one range split in nt equal parts, done by
+// the caller and nt - 1 worker threads (a pageable <-> pinned copy runs at 29 GB/s on one core, 76-80
+// GB/s on 4-8).
 // The workers start on the first use and live until the process ends (the pool is never destroyed,
 // so no thread can be waiting on a destroyed condition variable at exit).
 class CopyPool {
@@ -163,10 +164,11 @@ public:
     {
         for (int i = 1; i < nt_; i++) std::thread([this, i] { worker(i); }).detach();
     }
-    void copy(void *dst, const void *src, size_t n)
+    // dst = src, or (add: n and both addresses multiples of 4) dst += src as int32 modulo 2^32
+    void run(void *dst, const void *src, size_t n, bool add)
     {
         if (nt_ == 1 || n < ((size_t)1 << 20)) {
-            memcpy(dst, src, n);
+            range((uint8_t *)dst, (const uint8_t *)src, n, add);
             return;
         }
         {
@@ -174,6 +176,7 @@ public:
             dst_ = (uint8_t *)dst;
             src_ = (const uint8_t *)src;
             n_ = n;
+            add_ = add;
             pending_ = nt_ - 1;
             gen_++;
         }
@@ -188,7 +191,17 @@ private:
     {
         // ceil(n / nt) rounded up to 64 bytes: the nt parts cover all n bytes
         const size_t per = ((n_ + nt_ - 1) / nt_ + 63) & ~(size_t)63, b = std::min(n_, per * i), e = std::min(n_, b + per);
-        if (e > b) memcpy(dst_ + b, src_ + b, e - b);
+        if (e > b) range(dst_ + b, src_ + b, e - b, add_);
+    }
+    static void range(uint8_t *dst, const uint8_t *src, size_t n, bool add)
+    {
+        if (!add) {
+            memcpy(dst, src, n);
+            return;
+        }
+        uint32_t *d = (uint32_t *)dst;
+        const uint32_t *s = (const uint32_t *)src;
+        for (size_t i = 0; i < n / 4; i++) d[i] += s[i];
     }
     void worker(int i)
     {
@@ -212,23 +225,29 @@ private:
     uint8_t *dst_ = nullptr;
     const uint8_t *src_ = nullptr;
     size_t n_ = 0;
+    bool add_ = false;
 };
 
 // Device buffers, stream and pinned staging of the host-pointer GEMM (gemm_hip_i8 / gemm_ime_i8),
 // per device.  The device buffers only grow (hipMalloc of the larger size; the old one is freed,
 // which is safe because every call has synchronised its stream before returning) and are kept for
 // the life of the process, so a caller timing gemm_ime_i8 in a loop pays for the PCIe copies and
-// the kernel only.  The copies go through two pinned slots of HG_CHUNK bytes (hipHostMalloc, once):
-// the host copy of one chunk into (out of) a slot overlaps the DMA of the other slot, and pinned
-// DMA runs at about 57 GB/s where a pageable copy runs at 29 (H2D) and 18 GB/s (D2H).
-constexpr size_t HG_CHUNK = (size_t)8 << 20;
+// the kernel only.  C is not sent: the device computes A.B, and the host adds it to C as it comes back
+// (a pageable copy-out of the same bytes before), which leaves half of the traffic of C.  The copies go
+// through HG_SLOTS pinned slots of HG_CHUNK bytes (hipHostMalloc, once): the host's work on one chunk
+// overlaps the DMA of the others, and pinned DMA runs at about 57 GB/s where a pageable copy runs at 29
+// (H2D) and 18 GB/s (D2H).
+// 2048^3: 1098-1152 -> 663-760 us, 4096^3 3570-3780 -> 2360-2420, 64^3 60 -> 29 (chunks of 2 and 1 MiB 709
+// and 889 us at 2048^3, of 8 MiB 716 and 2266 at 4096^3 for twice the pinned memory; 8 threads no faster).
+constexpr size_t HG_CHUNK = (size_t)4 << 20;
+constexpr int HG_SLOTS = 4;
 struct HostGemmState {
     std::mutex mu;
     hipStream_t stream = nullptr;
     void *ab = nullptr, *c = nullptr;
     size_t ab_bytes = 0, c_bytes = 0;
-    void *pin[2] = {nullptr, nullptr};
-    hipEvent_t ev[2] = {nullptr, nullptr};
+    void *pin[HG_SLOTS] = {};
+    hipEvent_t ev[HG_SLOTS] = {};
     CopyPool *pool = nullptr;
 };
 HostGemmState g_host_gemm[64];
@@ -237,7 +256,7 @@ HostGemmState g_host_gemm[64];
 int host_gemm_setup(HostGemmState &h)
 {
     if (!h.stream) X100_TRY(hipStreamCreateWithFlags(&h.stream, hipStreamNonBlocking));
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < HG_SLOTS; i++) {
         if (!h.ev[i]) X100_TRY(hipEventCreateWithFlags(&h.ev[i], hipEventDisableTiming));
         if (!h.pin[i]) X100_TRY(hipHostMalloc(&h.pin[i], HG_CHUNK, hipHostMallocDefault));
     }
@@ -336,47 +355,42 @@ int gemm_hip_i8(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *
     if (rc) return rc;
     int8_t *dA = (int8_t *)h.ab, *dB = dA + sa;
     int32_t *dC = (int32_t *)h.c;
-    // A, B, C in: chunk i is copied into slot i % 2 once that slot's previous DMA is done, then
+    // A and B in: a chunk is copied into the next slot once that slot's previous DMA is done, then
     // DMA'd to the device.
     struct Piece {
         uint8_t *dev;
         const uint8_t *host;
         size_t bytes;
     };
-    const Piece in[3] = {{(uint8_t *)dA, (const uint8_t *)A, sa}, {(uint8_t *)dB, (const uint8_t *)B, sb},
-                         {(uint8_t *)dC, (const uint8_t *)C, sc}};
-    int slot = 0;
-    bool used[2] = {false, false};
+    const Piece in[2] = {{(uint8_t *)dA, (const uint8_t *)A, sa}, {(uint8_t *)dB, (const uint8_t *)B, sb}};
+    int n = 0;
     for (const Piece &pc : in)
-        for (size_t off = 0; off < pc.bytes; off += HG_CHUNK) {
+        for (size_t off = 0; off < pc.bytes; off += HG_CHUNK, n++) {
             const size_t len = std::min(HG_CHUNK, pc.bytes - off);
-            if (used[slot]) X100_TRY(hipEventSynchronize(h.ev[slot]));
-            h.pool->copy(h.pin[slot], pc.host + off, len);
+            const int slot = n % HG_SLOTS;
+            if (n >= HG_SLOTS) X100_TRY(hipEventSynchronize(h.ev[slot]));
+            h.pool->run(h.pin[slot], pc.host + off, len, false);
             X100_TRY(hipMemcpyAsync(pc.dev + off, h.pin[slot], len, hipMemcpyHostToDevice, h.stream));
             X100_TRY(hipEventRecord(h.ev[slot], h.stream));
-            used[slot] = true;
-            slot ^= 1;
         }
-    rc = gemm_hip_i8_dev(M, N, K, dA, dB, dC, h.stream);
+    rc = gemm_hip_i8_dev_set(M, N, K, dA, dB, dC, h.stream);
     if (rc != X100_OK) {
         (void)hipStreamSynchronize(h.stream);
         return rc;
     }
-    // C out: chunk i is DMA'd into slot i % 2 (after the kernel, in stream order) while the host
-    // copies chunk i - 1 out of the other slot.
+    // A.B out, up to HG_SLOTS chunks ahead (after the kernel, in stream order), each added to C as it
+    // arrives.
     const size_t nch = (sc + HG_CHUNK - 1) / HG_CHUNK;
-    for (size_t i = 0; i <= nch; i++) {
-        if (i < nch) {
-            const size_t len = std::min(HG_CHUNK, sc - i * HG_CHUNK);
-            X100_TRY(hipMemcpyAsync(h.pin[i & 1], (const uint8_t *)dC + i * HG_CHUNK, len, hipMemcpyDeviceToHost,
-                                    h.stream));
-            X100_TRY(hipEventRecord(h.ev[i & 1], h.stream));
+    size_t asked = 0;
+    for (size_t i = 0; i < nch; i++) {
+        for (; asked < nch && asked < i + HG_SLOTS; asked++) {
+            const int slot = (int)(asked % HG_SLOTS);
+            X100_TRY(hipMemcpyAsync(h.pin[slot], (const uint8_t *)dC + asked * HG_CHUNK,
+                                    std::min(HG_CHUNK, sc - asked * HG_CHUNK), hipMemcpyDeviceToHost, h.stream));
+            X100_TRY(hipEventRecord(h.ev[slot], h.stream));
         }
-        if (i > 0) {
-            const size_t j = i - 1, len = std::min(HG_CHUNK, sc - j * HG_CHUNK);
-            X100_TRY(hipEventSynchronize(h.ev[j & 1]));
-            h.pool->copy((uint8_t *)C + j * HG_CHUNK, h.pin[j & 1], len);
-        }
+        X100_TRY(hipEventSynchronize(h.ev[i % HG_SLOTS]));
+        h.pool->run((uint8_t *)C + i * HG_CHUNK, h.pin[i % HG_SLOTS], std::min(HG_CHUNK, sc - i * HG_CHUNK), true);
     }
     X100_TRY(hipStreamSynchronize(h.stream));
     return X100_OK;

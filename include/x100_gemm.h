@@ -26,8 +26,8 @@ extern "C" {
 #define X100_ENOMEM     -4   /* device allocation failed                               */
 
 /* Replaces gemm_ime_i8 (reference include/x100_gemm.h:60-61, src/gemm_ime_i8.c:60-89).  Host
- * pointers; copies A, B, C to the GPU, computes C += A*B there, copies C back and returns when C
- * is valid.  Same signature and void return as the reference; on failure it prints the reason
+ * pointers; copies A and B to the GPU, computes A*B there, adds it to C as it comes back and returns
+ * when C is valid.  Same signature and void return as the reference; on failure it prints the reason
  * to stderr and aborts (there is no CPU fallback).  The device buffers are allocated on the
  * first call, grow with the largest shape seen and are kept until the process ends; calls on one
  * device run one at a time (on a stream of the library's own, synchronised before returning). */

@@ -949,7 +949,7 @@ __host__ __device__ inline int mf_half(int nsb) { return nsb <= 4 ? nsb : min(ns
 inline size_t mf_lds(int nsb) { return (size_t)mf_half(nsb) * 8192 + (size_t)nsb * 512; }
 
 template <bool GU, bool TL, int RT>
-__global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, const uint8_t *__restrict__ Wa,
+__global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, int vr, const uint8_t *__restrict__ Wa,
                                                   const uint8_t *__restrict__ Wb, MoeWs ws)
 {
     // RT (down projection only, with every super-block staged at once): a wave walks RT tiles of
@@ -963,19 +963,30 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ int s_pairs[MF_PCH];
     __shared__ float s_dx[16][MF_PCH];          // activation scale [super-block][chunk pair]
-    __shared__ float s_up[GU ? 2 : 1][MF_PCH][33];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, col = lane & 31, h = lane >> 5;
-    // Blocks are dealt to the 8 XCDs round-robin; XCD x takes the chunks U x / 8 .. U (x + 1) / 8 - 1, one
-    // row range yb after the other, so that the chunks of one expert (adjacent) read the same weights
-    // at about the same time through one L2 (M = 512: the layer 173.8 -> 171.5 us).
-    const int U = *ws.nuniq, xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3;
-    const int u0 = U * xcd >> 3, per = (U * (xcd + 1) >> 3) - u0;
-    const int yb = local / max(per, 1), u = u0 + local - yb * per;
-    if (per == 0 || yb >= (GU ? ff / 64 : d / (128 * RT))) return;
-    // One round trip for the chunk's expert and size and its pair col (entries at or past the size
-    // are stale and replaced by pair 0, which every chunk has).
+    // Blocks are dealt to the 8 XCDs round-robin.  vr > 0: chunk = block modulo vr.  vr = 0 (experts with
+    // several chunks): XCD x takes the chunks U x / 8 .. U (x + 1) / 8 - 1, one row range yb after the
+    // other, so that the chunks of one expert (adjacent) read the same weights at about the same time
+    // through one L2 (M = 512: the layer 173.8 -> 171.5 us); that takes a round trip for U first (0.3
+    // us, more than it gives where most experts have one chunk).
+    const int U = *ws.nuniq;
+    int u, yb;
+    if (vr > 0) {
+        yb = (int)blockIdx.x / vr;
+        u = (int)blockIdx.x - yb * vr;
+    } else {
+        const int xcd = (int)blockIdx.x & 7, local = (int)blockIdx.x >> 3;
+        const int u0 = U * xcd >> 3, per = (U * (xcd + 1) >> 3) - u0;
+        yb = local / max(per, 1);
+        u = u0 + local - yb * per;
+        if (per == 0 || yb >= (GU ? ff / 64 : d / (128 * RT))) return;
+    }
+    // One round trip for the chunk's expert and size and its pair col (and U; u < the chunks at most keeps
+    // every index inside the workspace arrays; entries at or past the size are stale and replaced by
+    // pair 0, which every chunk has).
     const int ex = ws.uniq[u], cnt = ws.ucnt[u];
     int pc = ws.upairs[u * MF_PCH + col];
+    if (u >= U) return;
     pc = __shfl(pc, col < cnt ? lane : 0, 64);
     if (t < MF_PCH) s_pairs[t] = pc;
 
@@ -1014,7 +1025,12 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
     // DMA lane l fetches pair l % 32, bytes 16 * (l / 32) .. +16 of each sub-block.
     const uint8_t *src = X + (size_t)arow * rec + 16 * h;
     const int nh1 = mf_half(nsb);   // nsb, or even: the halves meet between two ring steps
-    // the sums per sub-block of pair t % 32: bytes {l_0..3, h_0..3, l_4..7, h_4..7} at [super-block][pair]
+    auto stage = [&](int sb0, int sb1) {
+        for (int c = 8 * sb0 + w; c < 8 * sb1; c += 4) dma_1k(src + 32 * c, smem + (c - 8 * sb0) * 1024);
+    };
+    stage(0, nh1);
+    // The sums per sub-block of pair t % 32: bytes {l_0..3, h_0..3, l_4..7, h_4..7} at [super-block][pair]
+    // (after the copies are requested: one round trip brings both).
     uint8_t *s_bs = smem + nh1 * 8192;
     for (int sb = t >> 5; sb < nsb; sb += 8) {
         const v4i *bp = (const v4i *)(X + (size_t)arow * rec + nsb * 256 + sb * 64);
@@ -1023,7 +1039,7 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
         for (int k = 0; k < 2; k++) {
             const v4i b0 = bp[2 * k], b1 = bp[2 * k + 1];
             const int s0 = b0[0] + b0[1], s1 = b0[2] + b0[3], s2 = b1[0] + b1[1], s3 = b1[2] + b1[3];
-            const uint32_t w01 = perm((uint32_t)s1, (uint32_t)s0, 0x05040100u) , w23 = perm((uint32_t)s3, (uint32_t)s2, 0x05040100u);
+            const uint32_t w01 = perm((uint32_t)s1, (uint32_t)s0, 0x05040100u), w23 = perm((uint32_t)s3, (uint32_t)s2, 0x05040100u);
             // 16-bit sums, two per dword: their low 6 bits, and the rest as signed bytes
             const uint32_t l01 = w01 & 0x003f003fu, l23 = w23 & 0x003f003fu;
             const uint32_t h01 = (w01 >> 6) & 0x00ff00ffu, h23 = (w23 >> 6) & 0x00ff00ffu;
@@ -1032,12 +1048,8 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
         }
         *(v4i *)(s_bs + (sb * 32 + col) * 16) = o;
     }
-    auto stage = [&](int sb0, int sb1) {
-        for (int c = 8 * sb0 + w; c < 8 * sb1; c += 4) dma_1k(src + 32 * c, smem + (c - 8 * sb0) * 1024);
-    };
-    stage(0, nh1);
     __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();   // staged activations, s_dx, s_pairs
+    __syncthreads();   // staged activations, s_bs, s_dx, s_pairs
 
     float acc[16];
 #pragma unroll
@@ -1124,6 +1136,10 @@ __global__ __launch_bounds__(256) void k_moe_mfma(int d, int ff, int n_act, cons
     }
 
     if constexpr (GU) {
+        // over the staged activations, which every wave has used: with LDS of its own, d = 3584 and 4096
+        // left room for one block per CU (M = 218, 16 experts: 205 us against 195 with two)
+        float(*s_up)[MF_PCH][33] = (float(*)[MF_PCH][33])smem;
+        __syncthreads();
         if (mat == 1)
 #pragma unroll
             for (int r = 0; r < 16; r++) s_up[w >> 1][8 * (r >> 2) + 4 * h + (r & 3)][col] = acc[r];
@@ -1493,19 +1509,21 @@ hipError_t moe_launch_mfma(int M, int d, int ff, int n_exp, int n_act, const flo
 {
     const int nsb = d / 256, nsf = ff / 256, P = M * n_act, nrc = (M + 7) / 8;
     const int Vmax = min(P, (P + MF_PCH - 1) / MF_PCH + n_exp), Vr = (Vmax + 7) & ~7;   // chunks at most
+    const int vr = P >= 24 * n_exp ? 0 : Vmax;   // block order (k_moe_mfma)
+    const int nc = vr ? Vmax : Vr;
     route_rows(M, d, n_exp, hn, R, ws, s);
     hipLaunchKernelGGL(k_moe_topk_rows, dim3(nrc), dim3(512), 0, s, M, n_exp, n_act, ws, sel, sw);
     hipLaunchKernelGGL(k_moe_group<MF_PCH>, dim3(1), dim3(256), 0, s, P, n_exp, ws);
-    hipLaunchKernelGGL((k_moe_mfma<true, TL, 1>), dim3(Vr * (ff / 64)), dim3(256), mf_lds(nsb), s, d,
-                       ff, n_act, (const uint8_t *)Wg, (const uint8_t *)Wu, ws);
+    hipLaunchKernelGGL((k_moe_mfma<true, TL, 1>), dim3(nc * (ff / 64)), dim3(256), mf_lds(nsb), s, d,
+                       ff, n_act, vr, (const uint8_t *)Wg, (const uint8_t *)Wu, ws);
     hipLaunchKernelGGL(k_moe_act_q8k, dim3((P * nsf + 3) / 4), dim3(256), 0, s, P, ff, ws);
     // down: MF_DN_RT row tiles per wave when one staging part holds every super-block
     if (MF_DN_RT > 1 && mf_half(nsf) == nsf && d % (128 * MF_DN_RT) == 0)
-        hipLaunchKernelGGL((k_moe_mfma<false, TL, MF_DN_RT>), dim3(Vr * (d / (128 * MF_DN_RT))), dim3(256),
-                           mf_lds(nsf), s, d, ff, n_act, (const uint8_t *)Wd, (const uint8_t *)nullptr, ws);
+        hipLaunchKernelGGL((k_moe_mfma<false, TL, MF_DN_RT>), dim3(nc * (d / (128 * MF_DN_RT))), dim3(256),
+                           mf_lds(nsf), s, d, ff, n_act, vr, (const uint8_t *)Wd, (const uint8_t *)nullptr, ws);
     else
-        hipLaunchKernelGGL((k_moe_mfma<false, TL, 1>), dim3(Vr * (d / 128)), dim3(256), mf_lds(nsf), s, d,
-                           ff, n_act, (const uint8_t *)Wd, (const uint8_t *)nullptr, ws);
+        hipLaunchKernelGGL((k_moe_mfma<false, TL, 1>), dim3(nc * (d / 128)), dim3(256), mf_lds(nsf), s, d,
+                           ff, n_act, vr, (const uint8_t *)Wd, (const uint8_t *)nullptr, ws);
     hipLaunchKernelGGL(k_moe_combine, dim3((M * d + 255) / 256), dim3(256), 0, s, M, d, n_act, ws, out, residual,
                        (const float *)nullptr);
     return hipGetLastError();

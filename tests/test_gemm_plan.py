@@ -1,0 +1,42 @@
+"""The int8 GEMM's kernel selection on the host (csrc/gemm_plan.h, compiled by tests/gemm_plan.cpp): at sizes
+too large to multiply in a test, no chosen kernel forms an offset that wraps."""
+import os
+import subprocess
+
+import pytest
+
+import x100hip
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(HERE, "..", "x100-gemm_amd", "csrc")
+VARIANTS = [x100hip.GEMM_AUTO, x100hip.GEMM_TILE256, x100hip.GEMM_TILE256_W4, x100hip.GEMM_TILE128, x100hip.GEMM_TILE64,
+            x100hip.GEMM_TILE32]
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("plan") / "gemm_plan")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-I", CSRC, os.path.join(HERE, "gemm_plan.cpp"), "-o", exe])
+
+    def ask(cases):   # (M, N, K, aligned, acc, variant) -> (kernel, tile, aligned, fits)
+        text = "".join("%d %d %d %d %d %d\n" % c for c in cases)
+        out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split("\n")
+        return [(k, t, int(a), int(f)) for k, t, a, f in (line.split() for line in out if line)]
+
+    return ask
+
+
+def test_wide_and_long_products_keep_their_offsets(plans):
+    edge = [7508480, 7508736, 1 << 23, (1 << 24) - 256, 1 << 24, 1 << 25, 1 << 27, (1 << 31) - 256]
+    cases = [(M, N, K, 1, acc, v) for v in VARIANTS for acc in (0, 1) for M in (48, 256, 512) for N in [4096] + edge
+             for K in [512, 576] + edge if N == 4096 or K <= 576]
+    for c, p in zip(cases, plans(cases)):
+        assert p[3] and p[0] != "refused", (c, p)
+
+
+def test_the_largest_256_tiles_stay(plans):
+    # the last sizes whose offsets fit still take k_gemm_big
+    cases = [(256, 7508480, 512, 1, 1, 1), (256, 1 << 27, 512, 1, 0, 1), (256, 512, 1 << 25, 1, 1, 1)]
+    assert [p[0] for p in plans(cases)] == ["big8"] * 3
+    cases = [(256, 7508736, 512, 1, 1, 1), (256, (1 << 27) + (1 << 26), 512, 1, 0, 1), (256, 512, 1 << 27, 1, 1, 1)]
+    assert not any(p[0] == "big8" for p in plans(cases))

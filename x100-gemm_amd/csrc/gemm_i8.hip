@@ -12,14 +12,11 @@
 //   k_gemm_skinny  M <= 16 rows (speculative-verify shapes): HBM-bound on B.  Split-K, B streamed
 //   (_mfma)        once through LDS, int32 atomics into C (exact and order independent).
 //   k_gemm_generic byte loads and scalar products: operands under 16 bytes, rows of 2^24 and more.
-#include <math.h>
-
+#include "gemm_plan.h"
 #include "x100_common.h"
 #include "x100_internal.h"
 
 namespace {
-
-constexpr int BK = 64;  // k bytes per pipeline stage
 
 // Tile order: blocks are dealt to the 8 XCDs round-robin, so block b runs on XCD b%8.  Give each
 // XCD a contiguous range of tile ids, and walk tile ids in groups of GROUP_M tile rows so the
@@ -57,7 +54,8 @@ X100_DEV void tile_coords(int bid, int nblk, int tiles_m, int tiles_n, int &tm, 
 // * C += A.B: the accumulators start at zero; the old C is prefetched a quarter of the tile at a
 //   time (before the K loop, then at 1/4, 1/2, 3/4 of it) and added when the next quarter is
 //   fetched, so C reads overlap the MFMA work.
-// Requires M % 256 == 0, N % 256 == 0, K % 64 == 0, K >= 512, 16-byte aligned pointers.
+// Requires M % 256 == 0, N % 256 == 0, K % 64 == 0, K >= 512, 16-byte aligned pointers, and K and N whose
+// 32-bit offsets below do not wrap (big_fits in gemm_plan.h).
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i lds_v2i;
@@ -149,14 +147,14 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_big(int M, int N, int K, const
     uint32_t aoff, boff;
     if constexpr (SUPER == 2) {
         const int ra = 8 * w + (lane >> 3);
-        aoff = (uint32_t)(ra * K + 16 * big_a2_chunk(ra, lane & 7));
+        aoff = (uint32_t)ra * (uint32_t)K + 16 * big_a2_chunk(ra, lane & 7);
     } else {
         const int ra = 16 * w + (lane >> 2);
-        aoff = (uint32_t)(ra * K + 16 * big_a_chunk(ra, lane & 3));
+        aoff = (uint32_t)ra * (uint32_t)K + 16 * big_a_chunk(ra, lane & 3);
     }
     {
         const int rb = 4 * w + (lane >> 4);
-        boff = (uint32_t)(rb * N + 16 * big_b_chunk(rb, lane & 15));
+        boff = (uint32_t)rb * (uint32_t)N + 16 * big_b_chunk(rb, lane & 15);
     }
     const uint32_t sbase = lds_addr(smem);
     auto dma_a = [&](const int8_t *ak, int p, uint32_t lds) __attribute__((always_inline)) {
@@ -207,7 +205,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_big(int M, int N, int K, const
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         const int r = 8 * t + (lane >> 3);
-        coff[t] = (uint32_t)(4 * ((wm * 128 + r) * N + wn * FN * 32 + 4 * big_a2_chunk(r, lane & 7)));
+        coff[t] = 4u * ((uint32_t)(wm * 128 + r) * (uint32_t)N + wn * FN * 32 + 4 * big_a2_chunk(r, lane & 7));
     }
     const uint32_t cl = lds_addr(csm) + (uint32_t)(w * 4096);
     auto load_c = [&](int p) __attribute__((always_inline)) {
@@ -1082,10 +1080,6 @@ __global__ __launch_bounds__(256) void k_gemm_generic(int M, int N, int K, const
         }
 }
 
-// Tiles of k_gemm_tile.  T128 (one block per CU), T64 and T32x64 and T32 (several); the unaligned
-// form takes 64x128 tiles of eight 32x32 waves in place of T128 (its staging registers).
-enum Tile { T128, T64, T32x64, T32, NTILE };
-
 template <int WM, int WN, int FM, int FN, int KW, bool ALN>
 hipError_t launch_tile_as(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C, hipStream_t s, bool acc)
 {
@@ -1117,78 +1111,13 @@ hipError_t launch_tile(Tile t, bool aln, int M, int N, int K, const int8_t *A, c
     }
 }
 
-// Estimated time (us) of a product on tile t: a start-up, C's traffic, and per 128-k stage the longer
-// of one block's own step (latency: few tiles) and the device's rate for all tiles (operand delivery
-// from L2, 12-16 TB/s: many tiles, which is why larger tiles win there).  Constants from graph
-// replays over M, N, K = 1 .. 4096 (us measured, T128 / T64 / T32x64 / T32, C = A.B):
-//   aligned   333x6144x2048  11.7 / 16.9 / 18.2 / 26.8    1024^3        7.7 / 5.6 / 6.2 / 8.3
-//             2048^3         15.0 / 23.6 / 29.8 / 47.3    17x4096x4096  15.1 / 7.1 / 6.4 / 6.6
-//             200x2048x2048   9.9 /  5.7 /  5.5 /  7.2    256^3         4.6 / 3.5 / 3.2 / 2.9
-//   unaligned 1001x1503x999  10.3 / 11.2 / 12.0 / 16.6    2047x300x2040 10.9 / 9.0 / 10.6 / 12.8
-//             33x2001x2001   13.5 / 10.1 /  8.3 /  7.3    37x41x257      5.4 / 4.3 / 4.1 / 3.6
-double c_us(int M, int N, bool acc) { return (double)M * N * (acc ? 8 : 4) / 6.5e6; }
-double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
-{
-    struct Cost {
-        int bm, bn;
-        double start, lat, thr;   // thr: a stage of 256 tiles
-    };
-    static const Cost costs[2][NTILE] = {
-        {{64, 128, 3.6, 0.60, 0.85}, {64, 64, 3.3, 0.38, 0.46}, {32, 64, 2.95, 0.33, 0.36}, {32, 32, 2.7, 0.25, 0.30}},
-        {{128, 128, 3.9, 0.35, 0.60}, {64, 64, 3.1, 0.12, 0.245}, {32, 64, 2.95, 0.10, 0.172}, {32, 32, 2.65, 0.095, 0.155}}};
-    const Cost &c = costs[aln][t];
-    const double tiles = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn), stages = (K + 127) / 128;
-    double per;
-    if (aln && t == T128) {   // one block per CU: whole rounds, and a last one that is at least a block's step
-        const double full = (double)((long)tiles / 256), rem = tiles - 256 * full;
-        per = full * c.thr + (rem > 0 ? fmax(c.lat, rem / 256 * c.thr) : 0.0);
-    } else {
-        per = fmax(c.lat, tiles / 256 * c.thr);
-    }
-    return c.start + c_us(M, N, acc) + per * stages;
-}
-Tile best_tile(bool aln, int M, int N, int K, bool acc, double &us)
-{
-    Tile best = T128;
-    us = tile_us(T128, aln, M, N, K, acc);
-    for (int t = T64; t < NTILE; t++) {
-        const double u = tile_us((Tile)t, aln, M, N, K, acc);
-        if (u < us) us = u, best = (Tile)t;
-    }
-    return best;
-}
-// k_gemm_big: rounds of 256 tiles, a last round no shorter than a block alone (4096^3 69.5 against 86
-// us on T128; 2048^2 x 4096, 64 tiles, 42 against 29).
-double big_us(int M, int N, int K, bool acc)
-{
-    const long tiles = (long)(M / 256) * (N / 256), full = tiles / 256, rem = tiles % 256;
-    return 3.0 + c_us(M, N, acc) + K / 128.0 * (full * 1.77 + (rem ? fmax(1.13, rem / 256.0 * 1.77) : 0.0));
-}
-// The split-K kernels for M <= 16 (C = A.B pays a clearing launch).  They stream B at up to 5 TB/s in
-// 128- or 256-column rows; the tiles reach 3.6 TB/s on a B beyond the caches, and less on rows that
-// are not whole cache lines (4x4112x4112: 7.0 us split-K, 9.4 on T32; 16x1280x1280: 7.7 and 3.7).
-double skinny_us(int M, int N, int K, bool acc)
-{
-    const double kn = (double)K * N, clear = acc ? 0.0 : 1.6;
-    if (N % 128 == 0 && K % 512 == 0) return clear + 2.9 + kn / 16e6;
-    return clear + (M <= 8 ? 4.7 + kn / 7e6 : 7.3 + kn / 4.3e6);
-}
-double skinny_tile_us(Tile &t, int M, int N, int K, bool acc)
-{
-    double us;
-    t = best_tile(true, M, N, K, acc, us);
-    if (N % 128) us = 2.65 + 1.5 * (us - 2.65);
-    return fmax(us, 2.65 + (double)K * N / 3.6e6);
-}
-
-// The 256x256 tile kernel k_gemm_big<NW, SUPER, ACC> (M, N multiples of 256, K % 64 == 0,
-// K >= 512); superstages when K / 64 is a multiple of 8 (the K shapes that path is tested on).
+// The 256x256 tile kernel k_gemm_big<NW, SUPER, ACC> (shapes of big_fits); superstages when K / 64 is a multiple of 8 (the K shapes that path is tested on).
 template <int NW>
 hipError_t launch_big(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C, hipStream_t s, bool acc)
 {
     const int tiles_m = M / 256, tiles_n = N / 256;
     const dim3 grid(tiles_m * tiles_n), block(NW * 64);
-    const bool super = (K / BK) % 8 == 0;
+    const bool super = big_super(K);
     if (super && acc)
         hipLaunchKernelGGL((k_gemm_big<NW, 2, true>), grid, block, 0, s, M, N, K, A, B, C, tiles_m, tiles_n);
     else if (super)
@@ -1232,38 +1161,12 @@ hipError_t x100_gemm_i8_launch(int M, int N, int K, const int8_t *A, const int8_
 {
     const bool aligned = (K % 16 == 0) && (N % 16 == 0) && (((uintptr_t)A & 15) == 0) &&
                          (((uintptr_t)B & 15) == 0) && (((uintptr_t)C & 15) == 0);
-    // k_gemm_tile: 32-bit offsets inside a tile and a stage, and a whole 16-byte chunk in each operand
-    const bool tiled = N < (1 << 24) && K < (1 << 24) && (size_t)M * K >= 16 && (size_t)K * N >= 16;
-    const bool whole = M % 256 == 0 && N % 256 == 0 && K % BK == 0 && K >= 512;   // k_gemm_big
-    Tile tile = T128;
-    if (variant == X100_GEMM_AUTO) {
-        double us = 0;
-        if (aligned && M <= 16 && (size_t)K * N < ((size_t)1 << 32) &&   // B must fit one buffer resource
-            (!tiled || skinny_us(M, N, K, acc) <= skinny_tile_us(tile, M, N, K, acc))) {
-            variant = X100_GEMM_SKINNY;
-        } else if (!tiled) {
-            variant = aligned && whole ? X100_GEMM_TILE256 : X100_GEMM_GENERIC;
-        } else {
-            tile = best_tile(aligned, M, N, K, acc, us);
-            if (!aligned || !whole || us < big_us(M, N, K, acc)) return launch_tile(tile, aligned, M, N, K, A, B, C, s, acc);
-            variant = X100_GEMM_TILE256;
-        }
-    }
-    if (!aligned && variant != X100_GEMM_GENERIC) return hipErrorInvalidValue;
-    const bool tile_variant = variant == X100_GEMM_TILE128 || variant == X100_GEMM_TILE64 || variant == X100_GEMM_TILE32 ||
-                              ((variant == X100_GEMM_TILE256 || variant == X100_GEMM_TILE256_W4) && !whole);
-    if (tile_variant && !tiled) variant = X100_GEMM_GENERIC;
-    switch (variant) {
-    case X100_GEMM_TILE256:
-        // Full 256x256 tiles only; other shapes use the 128x128 tile.
-        return whole ? launch_big<8>(M, N, K, A, B, C, s, acc) : launch_tile(T128, true, M, N, K, A, B, C, s, acc);
-    case X100_GEMM_TILE256_W4:
-        return whole ? launch_big<4>(M, N, K, A, B, C, s, acc) : launch_tile(T128, true, M, N, K, A, B, C, s, acc);
-    case X100_GEMM_TILE128: return launch_tile(T128, true, M, N, K, A, B, C, s, acc);
-    case X100_GEMM_TILE64: return launch_tile(T64, true, M, N, K, A, B, C, s, acc);
-    case X100_GEMM_TILE32: return launch_tile(T32, true, M, N, K, A, B, C, s, acc);
-    case X100_GEMM_SKINNY: {
-        if (M > 16 || (size_t)K * N >= ((size_t)1 << 32)) return hipErrorInvalidValue;
+    const GemmPlan plan = gemm_plan(M, N, K, aligned, acc, variant);
+    switch (plan.kernel) {
+    case GK_BIG8: return launch_big<8>(M, N, K, A, B, C, s, acc);
+    case GK_BIG4: return launch_big<4>(M, N, K, A, B, C, s, acc);
+    case GK_TILE: return launch_tile(plan.tile, plan.aligned, M, N, K, A, B, C, s, acc);
+    case GK_SKINNY: {
         if (!acc) {
             const hipError_t e = x100_zero_i32_launch(C, (size_t)M * N, s);
             if (e != hipSuccess) return e;
@@ -1279,7 +1182,7 @@ hipError_t x100_gemm_i8_launch(int M, int N, int K, const int8_t *A, const int8_
             hipLaunchKernelGGL((k_gemm_skinny<16, 4>), grid, dim3(256), 0, s, M, N, K, A, B, C);
         return hipGetLastError();
     }
-    case X100_GEMM_GENERIC: {
+    case GK_GENERIC: {
         dim3 grid((N + 63) / 64, (M + 63) / 64);
         if (acc)
             hipLaunchKernelGGL(k_gemm_generic<true>, grid, dim3(256), 0, s, M, N, K, A, B, C);
@@ -1287,6 +1190,7 @@ hipError_t x100_gemm_i8_launch(int M, int N, int K, const int8_t *A, const int8_
             hipLaunchKernelGGL(k_gemm_generic<false>, grid, dim3(256), 0, s, M, N, K, A, B, C);
         return hipGetLastError();
     }
+    case GK_REFUSED: break;
     }
     return hipErrorInvalidValue;
 }

@@ -1,0 +1,138 @@
+// Which kernel an int8 product takes: sizes and alignment only, on the host.  Plain C++ without HIP, so
+// that a test can evaluate it, with the kernels' 32-bit offsets, at sizes that no test multiplies.
+#pragma once
+#include <math.h>
+#include <stddef.h>
+#include <stdint.h>
+
+enum {
+    X100_GEMM_AUTO = 0,
+    X100_GEMM_TILE256 = 1,
+    X100_GEMM_TILE128 = 2,
+    X100_GEMM_SKINNY = 3,
+    X100_GEMM_GENERIC = 4,
+    X100_GEMM_TILE256_W4 = 5,   // 256x256 tile, 4 waves of 128x128
+    X100_GEMM_TILE64 = 6,       // 64x64 tile, 2 x 2 waves of 32x32, two groups on K
+    X100_GEMM_TILE32 = 7,       // 32x32 tile, four waves on K
+};
+
+// Tiles of k_gemm_tile.  T128 (one block per CU), T64 and T32x64 and T32 (several); the unaligned
+// form takes 64x128 tiles of eight 32x32 waves in place of T128 (its staging registers).
+enum Tile { T128, T64, T32x64, T32, NTILE };
+
+// Estimated time (us) of a product on tile t: a start-up, C's traffic, and per 128-k stage the longer
+// of one block's own step (latency: few tiles) and the device's rate for all tiles (operand delivery
+// from L2, 12-16 TB/s: many tiles, which is why larger tiles win there).  Constants from graph
+// replays over M, N, K = 1 .. 4096 (us measured, T128 / T64 / T32x64 / T32, C = A.B):
+//   aligned   333x6144x2048  11.7 / 16.9 / 18.2 / 26.8    1024^3        7.7 / 5.6 / 6.2 / 8.3
+//             2048^3         15.0 / 23.6 / 29.8 / 47.3    17x4096x4096  15.1 / 7.1 / 6.4 / 6.6
+//             200x2048x2048   9.9 /  5.7 /  5.5 /  7.2    256^3         4.6 / 3.5 / 3.2 / 2.9
+//   unaligned 1001x1503x999  10.3 / 11.2 / 12.0 / 16.6    2047x300x2040 10.9 / 9.0 / 10.6 / 12.8
+//             33x2001x2001   13.5 / 10.1 /  8.3 /  7.3    37x41x257      5.4 / 4.3 / 4.1 / 3.6
+inline double c_us(int M, int N, bool acc) { return (double)M * N * (acc ? 8 : 4) / 6.5e6; }
+inline double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
+{
+    struct Cost {
+        int bm, bn;
+        double start, lat, thr;   // thr: a stage of 256 tiles
+    };
+    static const Cost costs[2][NTILE] = {
+        {{64, 128, 3.6, 0.60, 0.85}, {64, 64, 3.3, 0.38, 0.46}, {32, 64, 2.95, 0.33, 0.36}, {32, 32, 2.7, 0.25, 0.30}},
+        {{128, 128, 3.9, 0.35, 0.60}, {64, 64, 3.1, 0.12, 0.245}, {32, 64, 2.95, 0.10, 0.172}, {32, 32, 2.65, 0.095, 0.155}}};
+    const Cost &c = costs[aln][t];
+    const double tiles = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn), stages = (K + 127) / 128;
+    double per;
+    if (aln && t == T128) {   // one block per CU: whole rounds, and a last one that is at least a block's step
+        const double full = (double)((long)tiles / 256), rem = tiles - 256 * full;
+        per = full * c.thr + (rem > 0 ? fmax(c.lat, rem / 256 * c.thr) : 0.0);
+    } else {
+        per = fmax(c.lat, tiles / 256 * c.thr);
+    }
+    return c.start + c_us(M, N, acc) + per * stages;
+}
+inline Tile best_tile(bool aln, int M, int N, int K, bool acc, double &us)
+{
+    Tile best = T128;
+    us = tile_us(T128, aln, M, N, K, acc);
+    for (int t = T64; t < NTILE; t++) {
+        const double u = tile_us((Tile)t, aln, M, N, K, acc);
+        if (u < us) us = u, best = (Tile)t;
+    }
+    return best;
+}
+// k_gemm_big: rounds of 256 tiles, a last round no shorter than a block alone (4096^3 69.5 against 86
+// us on T128; 2048^2 x 4096, 64 tiles, 42 against 29).
+inline double big_us(int M, int N, int K, bool acc)
+{
+    const long tiles = (long)(M / 256) * (N / 256), full = tiles / 256, rem = tiles % 256;
+    return 3.0 + c_us(M, N, acc) + K / 128.0 * (full * 1.77 + (rem ? fmax(1.13, rem / 256.0 * 1.77) : 0.0));
+}
+// The split-K kernels for M <= 16 (C = A.B pays a clearing launch).  They stream B at up to 5 TB/s in
+// 128- or 256-column rows; the tiles reach 3.6 TB/s on a B beyond the caches, and less on rows that
+// are not whole cache lines (4x4112x4112: 7.0 us split-K, 9.4 on T32; 16x1280x1280: 7.7 and 3.7).
+inline double skinny_us(int M, int N, int K, bool acc)
+{
+    const double kn = (double)K * N, clear = acc ? 0.0 : 1.6;
+    if (N % 128 == 0 && K % 512 == 0) return clear + 2.9 + kn / 16e6;
+    return clear + (M <= 8 ? 4.7 + kn / 7e6 : 7.3 + kn / 4.3e6);
+}
+inline double skinny_tile_us(Tile &t, int M, int N, int K, bool acc)
+{
+    double us;
+    t = best_tile(true, M, N, K, acc, us);
+    if (N % 128) us = 2.65 + 1.5 * (us - 2.65);
+    return fmax(us, 2.65 + (double)K * N / 3.6e6);
+}
+
+// k_gemm_big adds 32-bit byte offsets to 64-bit bases: up to row 127 of A (63 with superstages, K / 64 a
+// multiple of 8) and row 31 of B, and, where C is added, row 143 of C (4-byte elements).  Above these
+// sizes the offsets would wrap (C from N = 7.5 million columns).
+inline bool big_super(int K) { return K / 64 % 8 == 0; }
+inline uint64_t big_a_reach(int K) { return (big_super(K) ? 63ull : 127ull) * (uint64_t)K + 128; }
+inline uint64_t big_b_reach(int N) { return 31ull * (uint64_t)N + 256; }
+inline uint64_t big_c_reach(int N) { return 4 * (143ull * (uint64_t)N + 256); }
+inline bool big_fits(int M, int N, int K, bool acc)
+{
+    const uint64_t lim = (uint64_t)1 << 32;
+    return M % 256 == 0 && N % 256 == 0 && K % 64 == 0 && K >= 512 && big_a_reach(K) <= lim && big_b_reach(N) <= lim &&
+           (!acc || big_c_reach(N) <= lim);
+}
+
+enum GemmKernel { GK_REFUSED, GK_BIG8, GK_BIG4, GK_TILE, GK_SKINNY, GK_GENERIC };
+struct GemmPlan {
+    GemmKernel kernel;
+    Tile tile;      // GK_TILE
+    bool aligned;   // GK_TILE: the DMA form
+};
+
+// aligned: K, N multiples of 16 and A, B, C 16-byte aligned.  A forced variant other than the generic one
+// takes aligned operands only, and a forced 256x256 tile that the shape does not divide 128x128.
+inline GemmPlan gemm_plan(int M, int N, int K, bool aligned, bool acc, int variant)
+{
+    // k_gemm_tile: 32-bit offsets inside a tile and a stage, and a whole 16-byte chunk in each operand
+    const bool tiled = N < (1 << 24) && K < (1 << 24) && (size_t)M * K >= 16 && (size_t)K * N >= 16;
+    const bool whole = big_fits(M, N, K, acc);
+    const bool skinny = M <= 16 && (size_t)K * N < ((size_t)1 << 32);   // B must fit one buffer resource
+    auto on_tile = [&](Tile t) { return tiled ? GemmPlan{GK_TILE, t, aligned} : GemmPlan{GK_GENERIC, t, aligned}; };
+    if (variant != X100_GEMM_AUTO && variant != X100_GEMM_GENERIC && !aligned) return {GK_REFUSED, T128, false};
+    switch (variant) {
+    case X100_GEMM_AUTO: {
+        Tile t = T128;
+        double us = 0;
+        if (aligned && skinny && (!tiled || skinny_us(M, N, K, acc) <= skinny_tile_us(t, M, N, K, acc)))
+            return {GK_SKINNY, t, true};
+        if (!tiled) return {aligned && whole ? GK_BIG8 : GK_GENERIC, t, aligned};
+        t = best_tile(aligned, M, N, K, acc, us);
+        if (aligned && whole && us >= big_us(M, N, K, acc)) return {GK_BIG8, t, true};
+        return on_tile(t);
+    }
+    case X100_GEMM_TILE256: return whole ? GemmPlan{GK_BIG8, T128, true} : on_tile(T128);
+    case X100_GEMM_TILE256_W4: return whole ? GemmPlan{GK_BIG4, T128, true} : on_tile(T128);
+    case X100_GEMM_TILE128: return on_tile(T128);
+    case X100_GEMM_TILE64: return on_tile(T64);
+    case X100_GEMM_TILE32: return on_tile(T32);
+    case X100_GEMM_SKINNY: return {skinny ? GK_SKINNY : GK_REFUSED, T128, true};
+    case X100_GEMM_GENERIC: return {GK_GENERIC, T128, aligned};
+    }
+    return {GK_REFUSED, T128, false};
+}

@@ -3,19 +3,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gemm_plan.h"
 #include "x100_decode.h"
 #include "x100_moe.h"
-
-enum {
-    X100_GEMM_AUTO = 0,
-    X100_GEMM_TILE256 = 1,
-    X100_GEMM_TILE128 = 2,
-    X100_GEMM_SKINNY = 3,
-    X100_GEMM_GENERIC = 4,
-    X100_GEMM_TILE256_W4 = 5,   // 256x256 tile, 4 waves of 128x128
-    X100_GEMM_TILE64 = 6,       // 64x64 tile, 4 waves of 32x32
-    X100_GEMM_TILE32 = 7,       // 32x32 tile, 1 wave
-};
 
 // acc: C += A.B; otherwise the overwrite form C = A.B.
 hipError_t x100_gemm_i8_launch(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C,

@@ -34,7 +34,7 @@ static bool tile_offsets(int N, int K)
 
 int main()
 {
-    static const char *const kernels[] = {"refused", "big8", "big4", "tile", "skinny", "generic"};
+    static const char *const kernels[] = {"refused", "big8", "big4", "tile", "mfma", "skinny", "generic"};
     static const char *const tiles[] = {"128", "64", "32x64", "32"};
     int M, N, K, aligned, acc, variant;
     while (scanf("%d %d %d %d %d %d", &M, &N, &K, &aligned, &acc, &variant) == 6) {
@@ -42,7 +42,7 @@ int main()
         bool fits = true;
         if (p.kernel == GK_BIG8 || p.kernel == GK_BIG4) fits = big_offsets(p.kernel == GK_BIG8 ? 8 : 4, N, K, acc);
         if (p.kernel == GK_TILE) fits = tile_offsets(N, K);
-        printf("%s %s %d %d\n", kernels[p.kernel], p.kernel == GK_TILE ? tiles[p.tile] : "-", p.aligned, fits);
+        printf("%s %s %d %d\n", kernels[p.kernel], p.kernel == GK_TILE || p.kernel == GK_MFMA ? tiles[p.tile] : "-", p.aligned, fits);
     }
     return 0;
 }

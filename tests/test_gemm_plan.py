@@ -40,3 +40,11 @@ def test_the_largest_256_tiles_stay(plans):
     assert [p[0] for p in plans(cases)] == ["big8"] * 3
     cases = [(256, 7508736, 512, 1, 1, 1), (256, (1 << 27) + (1 << 26), 512, 1, 0, 1), (256, 512, 1 << 27, 1, 1, 1)]
     assert not any(p[0] == "big8" for p in plans(cases))
+
+
+def test_aligned_products_never_fall_to_the_scalar_kernel(plans):
+    sizes = [16, 48, 272, 512, 4096, (1 << 24) - 16, 1 << 24, (1 << 24) + 16, 1 << 28, (1 << 31) - 16]
+    cases = [(M, N, K, 1, acc, v) for v in VARIANTS for acc in (0, 1) for M in (1, 16, 17, 256, 1 << 24) for N in sizes
+             for K in sizes]
+    for c, p in zip(cases, plans(cases)):
+        assert p[0] not in ("generic", "refused") and p[3], (c, p)

@@ -9,9 +9,10 @@
 //                  reads for B, v_mfma_i32_32x32x32_i8.
 //   k_gemm_tile    tiles from 32x32 to 128x128 for every other shape and alignment, same operand
 //                  path in a 4-slot ring of 128-k stages (unaligned operands through registers).
+//   k_gemm_mfma    aligned tiles of 64-k stages through registers: N or K of 2^24 and more.
 //   k_gemm_skinny  M <= 16 rows (speculative-verify shapes): HBM-bound on B.  Split-K, B streamed
 //   (_mfma)        once through LDS, int32 atomics into C (exact and order independent).
-//   k_gemm_generic byte loads and scalar products: operands under 16 bytes, rows of 2^24 and more.
+//   k_gemm_generic byte loads and scalar products: operands under 16 bytes, unaligned rows of 2^24 and more.
 #include "gemm_plan.h"
 #include "x100_common.h"
 #include "x100_internal.h"
@@ -33,6 +34,164 @@ X100_DEV void tile_coords(int bid, int nblk, int tiles_m, int tiles_n, int &tm, 
     int r = t - g * per_group;
     tm = first_m + r % gsize;
     tn = r / gsize;
+}
+
+// ------------------------------------------------------------------------------------------------
+// k_gemm_mfma: tiles of 64-k stages through registers into two LDS buffers (A in 16-byte chunks, B
+// transposed in registers into dwords of four consecutive k of one column).  Offsets are 64-bit and an
+// index past the end is compared as unsigned: any M, N and K of aligned operands.
+// ------------------------------------------------------------------------------------------------
+constexpr int BK = 64;   // k bytes per stage
+
+// A tile in LDS: BM rows x 64 bytes; 16-byte chunk c of row r stored at chunk c ^ ((r>>1)&3)
+// so that 8 consecutive lanes reading one chunk column hit 8 distinct 16-byte bank groups.
+X100_DEV int a_lds_off(int r, int c) { return r * BK + ((c ^ ((r >> 1) & 3)) << 4); }
+
+template <int FM, int FN, int WM, int WN, bool EDGE, bool ACC>
+__global__ __launch_bounds__(WM *WN * 64) void k_gemm_mfma(int M, int N, int K,
+                                                           const int8_t *__restrict__ A,
+                                                           const int8_t *__restrict__ B,
+                                                           int32_t *__restrict__ C, int tiles_m,
+                                                           int tiles_n)
+{
+    constexpr int NT = WM * WN * 64;
+    constexpr int BM = WM * FM * 32;
+    constexpr int BN = WN * FN * 32;
+    constexpr int A_IT = BM * 4 / NT;             // 16-byte A chunks per thread per stage
+    constexpr int B_UNITS = BN;                   // (k-quad, 16 columns) units per stage
+    constexpr int B_IT = (B_UNITS + NT - 1) / NT;
+    static_assert(A_IT * NT == BM * 4, "A tile must split evenly over the threads");
+
+    __shared__ __attribute__((aligned(16))) int8_t As[2][BM * BK];
+    __shared__ __attribute__((aligned(16))) uint32_t Bs[2][16 * BN];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave / WN, wn = wave % WN;
+    const int lcol = lane & 31, lgrp = lane >> 5;
+    int tm, tn;
+    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+    // EDGE = false is only launched when M % BM == 0, N % BN == 0 and K % BK == 0.
+    const bool full_mn = !EDGE || (M - m0 >= BM && N - n0 >= BN);
+    auto in = [](int i, int n) { return (uint32_t)i < (uint32_t)n; };
+
+    // Accumulators start from C (ACC: C += A.B) or from zero (C = A.B, C never read).  32x32 MFMA
+    // output layout: lane l, register r holds row 8*(r/4) + 4*(l/32) + r%4, column l%32.
+    v16i acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            const int gn = n0 + wn * FN * 32 + 32 * j + lcol;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int gm = m0 + wm * FM * 32 + 32 * i + 8 * (r >> 2) + 4 * lgrp + (r & 3);
+                acc[i][j][r] = (ACC && (full_mn || (in(gm, M) && in(gn, N)))) ? C[(size_t)gm * N + gn] : 0;
+            }
+        }
+
+    v4i ra[A_IT];
+    v4i rb[B_IT][4];
+
+    auto gload = [&](int kt) {
+        const int k0 = kt * BK;
+        const bool full = !EDGE || (full_mn && K - k0 >= BK);
+#pragma unroll
+        for (int p = 0; p < A_IT; p++) {
+            const int ch = tid + p * NT, r = ch >> 2, c = ch & 3;
+            const int gm = m0 + r, gk = k0 + 16 * c;
+            if (full || (in(gm, M) && in(gk, K)))
+                ra[p] = *(const v4i *)(A + (size_t)gm * K + gk);
+            else
+                ra[p] = v4i{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int p = 0; p < B_IT; p++) {
+            const int u = tid + p * NT;
+            if (B_UNITS % NT == 0 || u < B_UNITS) {
+                const int kq = u / (BN / 16), nc = u % (BN / 16);
+                const int gn = n0 + 16 * nc;
+#pragma unroll
+                for (int rr = 0; rr < 4; rr++) {
+                    const int gk = k0 + 4 * kq + rr;
+                    if (full || (in(gk, K) && in(gn, N)))
+                        rb[p][rr] = *(const v4i *)(B + (size_t)gk * N + gn);
+                    else
+                        rb[p][rr] = v4i{0, 0, 0, 0};
+                }
+            }
+        }
+    };
+
+    auto lstore = [&](int buf) {
+#pragma unroll
+        for (int p = 0; p < A_IT; p++) {
+            const int ch = tid + p * NT, r = ch >> 2, c = ch & 3;
+            *(v4i *)(&As[buf][a_lds_off(r, c)]) = ra[p];
+        }
+#pragma unroll
+        for (int p = 0; p < B_IT; p++) {
+            const int u = tid + p * NT;
+            if (B_UNITS % NT == 0 || u < B_UNITS) {
+                const int kq = u / (BN / 16), nc = u % (BN / 16);
+                uint32_t o[16];
+#pragma unroll
+                for (int cg = 0; cg < 4; cg++)
+                    transpose4x4((uint32_t)rb[p][0][cg], (uint32_t)rb[p][1][cg],
+                                 (uint32_t)rb[p][2][cg], (uint32_t)rb[p][3][cg], o[4 * cg + 0],
+                                 o[4 * cg + 1], o[4 * cg + 2], o[4 * cg + 3]);
+                v4u *dst = (v4u *)(&Bs[buf][kq * BN + 16 * nc]);
+                dst[0] = v4u{o[0], o[1], o[2], o[3]};
+                dst[1] = v4u{o[4], o[5], o[6], o[7]};
+                dst[2] = v4u{o[8], o[9], o[10], o[11]};
+                dst[3] = v4u{o[12], o[13], o[14], o[15]};
+            }
+        }
+    };
+
+    const int nk = (K - 1) / BK + 1;
+    gload(0);
+    lstore(0);
+    __syncthreads();
+    for (int kt = 0; kt < nk; kt++) {
+        const int buf = kt & 1;
+        if (kt + 1 < nk) gload(kt + 1);
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            v4i af[FM], bf[FN];
+#pragma unroll
+            for (int i = 0; i < FM; i++) {
+                const int r = wm * FM * 32 + 32 * i + lcol;
+                af[i] = *(const v4i *)(&As[buf][a_lds_off(r, 2 * kk + lgrp)]);
+            }
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                const int n = wn * FN * 32 + 32 * j + lcol;
+                const int kq = 8 * kk + 4 * lgrp;
+                const uint32_t *bp = &Bs[buf][kq * BN + n];
+                bf[j] = v4i{(int)bp[0], (int)bp[BN], (int)bp[2 * BN], (int)bp[3 * BN]};
+            }
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
+        }
+        if (kt + 1 < nk) lstore(buf ^ 1);
+        __syncthreads();
+    }
+
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            const int gn = n0 + wn * FN * 32 + 32 * j + lcol;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int gm = m0 + wm * FM * 32 + 32 * i + 8 * (r >> 2) + 4 * lgrp + (r & 3);
+                if (full_mn || (in(gm, M) && in(gn, N))) C[(size_t)gm * N + gn] = acc[i][j][r];
+            }
+        }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -509,7 +668,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_big(int M, int N, int K, const
 //   64 x 64 tiles: 17.5 us with fragments read and used in the same stage, 13.1, 11.9, 10.7).
 // * C is read (ACC) first and written as dwords (32 lanes = one 128-byte row segment): any alignment.
 // Bound by operand delivery (L2 to LDS, 12-16 TB/s over the chip) with many tiles and by the stage's
-// latency with few.  In place of register-staged 64-k tiles and of scalar products on unaligned
+// latency with few.  In place of k_gemm_mfma's tiles and of scalar products on unaligned
 // shapes: 333 x 6144 x 2048 26.7 -> 11.7 us, 2048^3 24.3 -> 15.0, 1001 x 1503 x 999 178 -> 10.3.
 // ------------------------------------------------------------------------------------------------
 typedef int v4i_u __attribute__((ext_vector_type(4), aligned(1)));
@@ -1111,6 +1270,21 @@ hipError_t launch_tile(Tile t, bool aln, int M, int N, int K, const int8_t *A, c
     }
 }
 
+template <int FM, int FN, int WM, int WN>
+hipError_t launch_mfma(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C, hipStream_t s, bool acc)
+{
+    constexpr int BM = WM * FM * 32, BN = WN * FN * 32;
+    const int tiles_m = (M - 1) / BM + 1, tiles_n = (N - 1) / BN + 1;
+    const dim3 grid(tiles_m * tiles_n), block(WM * WN * 64);
+    auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, block, 0, s, M, N, K, A, B, C, tiles_m, tiles_n); };
+    const bool edge = (M % BM) || (N % BN) || (K % BK);
+    if (edge && acc) go(k_gemm_mfma<FM, FN, WM, WN, true, true>);
+    else if (edge) go(k_gemm_mfma<FM, FN, WM, WN, true, false>);
+    else if (acc) go(k_gemm_mfma<FM, FN, WM, WN, false, true>);
+    else go(k_gemm_mfma<FM, FN, WM, WN, false, false>);
+    return hipGetLastError();
+}
+
 // The 256x256 tile kernel k_gemm_big<NW, SUPER, ACC> (shapes of big_fits); superstages when K / 64 is a multiple of 8 (the K shapes that path is tested on).
 template <int NW>
 hipError_t launch_big(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C, hipStream_t s, bool acc)
@@ -1166,6 +1340,10 @@ hipError_t x100_gemm_i8_launch(int M, int N, int K, const int8_t *A, const int8_
     case GK_BIG8: return launch_big<8>(M, N, K, A, B, C, s, acc);
     case GK_BIG4: return launch_big<4>(M, N, K, A, B, C, s, acc);
     case GK_TILE: return launch_tile(plan.tile, plan.aligned, M, N, K, A, B, C, s, acc);
+    case GK_MFMA:
+        return plan.tile == T128 ? launch_mfma<2, 2, 2, 2>(M, N, K, A, B, C, s, acc)
+               : plan.tile == T64 ? launch_mfma<1, 1, 2, 2>(M, N, K, A, B, C, s, acc)
+                                  : launch_mfma<1, 1, 1, 1>(M, N, K, A, B, C, s, acc);
     case GK_SKINNY: {
         if (!acc) {
             const hipError_t e = x100_zero_i32_launch(C, (size_t)M * N, s);

@@ -40,7 +40,7 @@ inline double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
         {{64, 128, 3.6, 0.60, 0.85}, {64, 64, 3.3, 0.38, 0.46}, {32, 64, 2.95, 0.33, 0.36}, {32, 32, 2.7, 0.25, 0.30}},
         {{128, 128, 3.9, 0.35, 0.60}, {64, 64, 3.1, 0.12, 0.245}, {32, 64, 2.95, 0.10, 0.172}, {32, 32, 2.65, 0.095, 0.155}}};
     const Cost &c = costs[aln][t];
-    const double tiles = (double)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn), stages = (K + 127) / 128;
+    const double tiles = (double)((M - 1) / c.bm + 1) * ((N - 1) / c.bn + 1), stages = (K - 1) / 128 + 1;
     double per;
     if (aln && t == T128) {   // one block per CU: whole rounds, and a last one that is at least a block's step
         const double full = (double)((long)tiles / 256), rem = tiles - 256 * full;
@@ -98,10 +98,18 @@ inline bool big_fits(int M, int N, int K, bool acc)
            (!acc || big_c_reach(N) <= lim);
 }
 
-enum GemmKernel { GK_REFUSED, GK_BIG8, GK_BIG4, GK_TILE, GK_SKINNY, GK_GENERIC };
+// k_gemm_mfma's tile by output size.  1024^2 x 4096 took 27.3 us on 64x64 tiles and 39.9 on 128x128, 2048^2 x
+// 4096 52.6 on 128x128; 256^3 3.5 on 32x32 and 5.7 on 128x128.
+inline Tile mfma_tile(int M, int N)
+{
+    const double mn = (double)M * N;
+    return mn >= 4.0 * 1024 * 1024 ? T128 : mn >= 1024.0 * 1024 ? T64 : T32;
+}
+
+enum GemmKernel { GK_REFUSED, GK_BIG8, GK_BIG4, GK_TILE, GK_MFMA, GK_SKINNY, GK_GENERIC };
 struct GemmPlan {
     GemmKernel kernel;
-    Tile tile;      // GK_TILE
+    Tile tile;      // GK_TILE, GK_MFMA (T128, T64 or T32)
     bool aligned;   // GK_TILE: the DMA form
 };
 
@@ -109,11 +117,12 @@ struct GemmPlan {
 // takes aligned operands only, and a forced 256x256 tile that the shape does not divide 128x128.
 inline GemmPlan gemm_plan(int M, int N, int K, bool aligned, bool acc, int variant)
 {
-    // k_gemm_tile: 32-bit offsets inside a tile and a stage, and a whole 16-byte chunk in each operand
+    // k_gemm_tile: 32-bit offsets inside a tile and a stage, and a whole 16-byte chunk in each operand; past them
+    // k_gemm_mfma takes aligned operands (33 x 2^24 x 400 2.4-3.5 ms, on the generic kernel 20.6-20.9)
     const bool tiled = N < (1 << 24) && K < (1 << 24) && (size_t)M * K >= 16 && (size_t)K * N >= 16;
     const bool whole = big_fits(M, N, K, acc);
     const bool skinny = M <= 16 && (size_t)K * N < ((size_t)1 << 32);   // B must fit one buffer resource
-    auto on_tile = [&](Tile t) { return tiled ? GemmPlan{GK_TILE, t, aligned} : GemmPlan{GK_GENERIC, t, aligned}; };
+    auto on_tile = [&](Tile t) { return GemmPlan{tiled ? GK_TILE : aligned ? GK_MFMA : GK_GENERIC, t, aligned}; };
     if (variant != X100_GEMM_AUTO && variant != X100_GEMM_GENERIC && !aligned) return {GK_REFUSED, T128, false};
     switch (variant) {
     case X100_GEMM_AUTO: {
@@ -121,7 +130,7 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool aligned, bool acc, int varia
         double us = 0;
         if (aligned && skinny && (!tiled || skinny_us(M, N, K, acc) <= skinny_tile_us(t, M, N, K, acc)))
             return {GK_SKINNY, t, true};
-        if (!tiled) return {aligned && whole ? GK_BIG8 : GK_GENERIC, t, aligned};
+        if (!tiled) return aligned && whole ? GemmPlan{GK_BIG8, t, true} : on_tile(mfma_tile(M, N));
         t = best_tile(aligned, M, N, K, acc, us);
         if (aligned && whole && us >= big_us(M, N, K, acc)) return {GK_BIG8, t, true};
         return on_tile(t);

@@ -32,6 +32,16 @@ static bool tile_offsets(int N, int K)
     return same(127u * (uint32_t)K + 128, 127ull * K + 128) && same(127u * (uint32_t)N + 128, 127ull * N + 128);
 }
 
+// Threads of the launch, 256x256 and split-K kernels aside (their C or B cannot be large enough).
+static bool launches(const GemmPlan &p, int M, int N)
+{
+    static const int bm[] = {128, 64, 32, 32}, bn[] = {128, 64, 64, 32};
+    const bool mfma = p.kernel == GK_MFMA;
+    const uint64_t rows = p.kernel == GK_TILE && p.tile == T128 && !p.aligned ? 64 : bm[p.tile];
+    const uint64_t nt = mfma ? (p.tile == T32 ? 64 : 256) : p.tile == T128 ? 512 : 256;
+    return ((M - 1) / rows + 1) * ((N - 1) / (uint64_t)bn[p.tile] + 1) * nt <= 0xffffffffu;
+}
+
 int main()
 {
     static const char *const kernels[] = {"refused", "big8", "big4", "tile", "mfma", "skinny", "generic"};
@@ -41,7 +51,8 @@ int main()
         const GemmPlan p = gemm_plan(M, N, K, aligned, acc, variant);
         bool fits = true;
         if (p.kernel == GK_BIG8 || p.kernel == GK_BIG4) fits = big_offsets(p.kernel == GK_BIG8 ? 8 : 4, N, K, acc);
-        if (p.kernel == GK_TILE) fits = tile_offsets(N, K);
+        if (p.kernel == GK_TILE) fits = tile_offsets(N, K) && launches(p, M, N);
+        if (p.kernel == GK_MFMA) fits = launches(p, M, N);
         printf("%s %s %d %d\n", kernels[p.kernel], p.kernel == GK_TILE || p.kernel == GK_MFMA ? tiles[p.tile] : "-", p.aligned, fits);
     }
     return 0;

@@ -19,17 +19,21 @@ def plans(tmp_path_factory):
     subprocess.check_call(["g++", "-O2", "-std=c++17", "-I", CSRC, os.path.join(HERE, "gemm_plan.cpp"), "-o", exe])
 
     def ask(cases):   # (M, N, K, aligned, acc, variant) -> (kernel, tile, aligned, fits)
-        text = "".join("%d %d %d %d %d %d\n" % c for c in cases)
+        text = "".join("%d %d %d %d %d %d\n" % tuple(map(int, c)) for c in cases)
         out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True).stdout.split("\n")
         return [(k, t, int(a), int(f)) for k, t, a, f in (line.split() for line in out if line)]
 
     return ask
 
 
+def exists(M, N, K):   # operands that fit one device
+    return M * N * 4 + M * K + K * N < 288e9
+
+
 def test_wide_and_long_products_keep_their_offsets(plans):
     edge = [7508480, 7508736, 1 << 23, (1 << 24) - 256, 1 << 24, 1 << 25, 1 << 27, (1 << 31) - 256]
     cases = [(M, N, K, 1, acc, v) for v in VARIANTS for acc in (0, 1) for M in (48, 256, 512) for N in [4096] + edge
-             for K in [512, 576] + edge if N == 4096 or K <= 576]
+             for K in [512, 576] + edge if exists(M, N, K)]
     for c, p in zip(cases, plans(cases)):
         assert p[3] and p[0] != "refused", (c, p)
 
@@ -45,6 +49,16 @@ def test_the_largest_256_tiles_stay(plans):
 def test_aligned_products_never_fall_to_the_scalar_kernel(plans):
     sizes = [16, 48, 272, 512, 4096, (1 << 24) - 16, 1 << 24, (1 << 24) + 16, 1 << 28, (1 << 31) - 16]
     cases = [(M, N, K, 1, acc, v) for v in VARIANTS for acc in (0, 1) for M in (1, 16, 17, 256, 1 << 24) for N in sizes
-             for K in sizes]
+             for K in sizes if exists(M, N, K)]
     for c, p in zip(cases, plans(cases)):
         assert p[0] not in ("generic", "refused") and p[3], (c, p)
+
+
+def test_tall_products_launch(plans):
+    # one column of tiles: the grid of every plan holds at most 2^32 - 1 threads
+    cases = [(M, N, K, K % 16 == 0 and N % 16 == 0, acc, 0) for acc in (0, 1) for K in (15, 16) for N in (1, 15, 16, 32, 48, 64)
+             for M in ((1 << 29) - 32, 1 << 29, (1 << 30) - 128, 1 << 30, (1 << 30) + 1, (1 << 31) - 256) if exists(M, N, K)]
+    got = plans(cases)
+    for c, p in zip(cases, got):
+        assert p[3] and p[0] != "refused" and (p[0] != "generic" or not c[3]), (c, p)
+    assert any(p[0] == "mfma" for p in got) and any(p[0] == "generic" for p in got)

@@ -53,3 +53,8 @@ def test_rows_of_2_24(dev, M, N, K, variants):
     for variant in variants:   # AUTO, TILE128, TILE64, TILE32
         for acc in (True, False):
             check(dev, M, N, K, acc, variant)
+
+
+# more rows than one launch of k_gemm_tile holds (2^32 - 1 threads)
+def test_2_30_rows(dev):
+    check(dev, (1 << 30) + 33, 16, 16, True)

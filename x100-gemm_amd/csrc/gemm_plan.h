@@ -106,6 +106,14 @@ inline Tile mfma_tile(int M, int N)
     return mn >= 4.0 * 1024 * 1024 ? T128 : mn >= 1024.0 * 1024 ? T64 : T32;
 }
 
+// Threads of a launch of k_gemm_tile: the runtime takes at most 2^32 - 1 (one column of tiles reaches that at
+// M = 2^30, where k_gemm_mfma's 128x128 tiles, 256 threads each, and the generic kernel's grid do not).
+inline bool tile_launches(Tile t, bool aln, int M, int N)
+{
+    const uint64_t bm = t == T128 ? (aln ? 128 : 64) : t == T64 ? 64 : 32, bn = t == T128 ? 128 : t == T32 ? 32 : 64;
+    return (((uint64_t)M - 1) / bm + 1) * (((uint64_t)N - 1) / bn + 1) * (t == T128 ? 512 : 256) < ((uint64_t)1 << 32);
+}
+
 enum GemmKernel { GK_REFUSED, GK_BIG8, GK_BIG4, GK_TILE, GK_MFMA, GK_SKINNY, GK_GENERIC };
 struct GemmPlan {
     GemmKernel kernel;
@@ -122,7 +130,9 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool aligned, bool acc, int varia
     const bool tiled = N < (1 << 24) && K < (1 << 24) && (size_t)M * K >= 16 && (size_t)K * N >= 16;
     const bool whole = big_fits(M, N, K, acc);
     const bool skinny = M <= 16 && (size_t)K * N < ((size_t)1 << 32);   // B must fit one buffer resource
-    auto on_tile = [&](Tile t) { return GemmPlan{tiled ? GK_TILE : aligned ? GK_MFMA : GK_GENERIC, t, aligned}; };
+    auto on_tile = [&](Tile t) {
+        return GemmPlan{tiled && tile_launches(t, aligned, M, N) ? GK_TILE : aligned ? GK_MFMA : GK_GENERIC, t, aligned};
+    };
     if (variant != X100_GEMM_AUTO && variant != X100_GEMM_GENERIC && !aligned) return {GK_REFUSED, T128, false};
     switch (variant) {
     case X100_GEMM_AUTO: {
@@ -133,7 +143,7 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool aligned, bool acc, int varia
         if (!tiled) return aligned && whole ? GemmPlan{GK_BIG8, t, true} : on_tile(mfma_tile(M, N));
         t = best_tile(aligned, M, N, K, acc, us);
         if (aligned && whole && us >= big_us(M, N, K, acc)) return {GK_BIG8, t, true};
-        return on_tile(t);
+        return on_tile(tile_launches(t, aligned, M, N) ? t : mfma_tile(M, N));
     }
     case X100_GEMM_TILE256: return whole ? GemmPlan{GK_BIG8, T128, true} : on_tile(T128);
     case X100_GEMM_TILE256_W4: return whole ? GemmPlan{GK_BIG4, T128, true} : on_tile(T128);

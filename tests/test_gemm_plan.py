@@ -27,7 +27,7 @@ def plans(tmp_path_factory):
 
 
 def exists(M, N, K):   # operands that fit one device
-    return M * N * 4 + M * K + K * N < 288e9
+    return M * N * 4 + M * K + K * N < 200e9
 
 
 def test_wide_and_long_products_keep_their_offsets(plans):
@@ -49,7 +49,7 @@ def test_the_largest_256_tiles_stay(plans):
 def test_aligned_products_never_fall_to_the_scalar_kernel(plans):
     sizes = [16, 48, 272, 512, 4096, (1 << 24) - 16, 1 << 24, (1 << 24) + 16, 1 << 28, (1 << 31) - 256]
     cases = [(M, N, K, 1, acc, v) for v in VARIANTS for acc in (0, 1) for M in (1, 16, 17, 256, 1 << 24) for N in sizes
-             for K in sizes if exists(M, N, K)]
+             for K in sizes if exists(M, N, K) and (v == x100hip.GEMM_AUTO or N <= 1 << 28)]
     for c, p in zip(cases, plans(cases)):
         assert p[0] not in ("generic", "refused") and p[3], (c, p)
 

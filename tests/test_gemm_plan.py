@@ -62,3 +62,21 @@ def test_tall_products_launch(plans):
     for c, p in zip(cases, got):
         assert p[3] and p[0] != "refused" and (p[0] != "generic" or not c[3]), (c, p)
     assert any(p[0] == "mfma" for p in got) and any(p[0] == "generic" for p in got)
+
+
+def test_short_k_takes_the_kernel_with_several_blocks_per_cu(plans):
+    from test_gemm_short_k_gpu import SHAPES
+    got = {(M, N, K, acc): p[:2] for (M, N, K, _, acc, _), p in zip(
+        [s + (1, acc, 0) for s in SHAPES for acc in (0, 1)], plans([s + (1, acc, 0) for s in SHAPES for acc in (0, 1)]))}
+    for acc in (0, 1):   # both tiles, whole and ragged, are among the GPU test's sizes
+        assert {k[:3] for k, p in got.items() if k[3] == acc and p == ("mfma", "128")} >= {(2048, 2176, 64), (2049, 2128, 80),
+                                                                                        (4096, 1152, 192), (8000, 4112, 176)}
+        assert {k[:3] for k, p in got.items() if k[3] == acc and p == ("mfma", "64")} >= {(1024, 1024, 64), (1601, 1040, 48),
+                                                                                       (64, 65536, 64), (70001, 32, 64)}
+    # sizes that were 1.1 to 1.6 times slower on k_gemm_tile
+    slow = [(4096, 4096, 64, 1), (4096, 4096, 256, 0), (4096, 4096, 256, 1), (7168, 4096, 320, 1), (256, 1 << 20, 128, 0), (16384, 16384, 256, 0), (65536, 256, 128, 1)]
+    assert {p[0] for p in plans([(M, N, K, 1, acc, 0) for M, N, K, acc in slow])} == {"mfma"}
+    # and sizes that are faster there
+    fast = [(333, 6144, 2048, 0), (256, 256, 256, 1), (2000, 8128, 512, 1), (512, 512, 64, 0), (31, 209280, 128, 1),
+            (35584, 192, 128, 1), (1024, 3584, 384, 0)]
+    assert {p[0] for p in plans([(M, N, K, 1, acc, 0) for M, N, K, acc in fast])} == {"tile"}

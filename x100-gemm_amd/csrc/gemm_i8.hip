@@ -9,7 +9,8 @@
 //                  reads for B, v_mfma_i32_32x32x32_i8.
 //   k_gemm_tile    tiles from 32x32 to 128x128 for every other shape and alignment, same operand
 //                  path in a 4-slot ring of 128-k stages (unaligned operands through registers).
-//   k_gemm_mfma    aligned tiles of 64-k stages through registers: N or K of 2^24 and more.
+//   k_gemm_mfma    aligned tiles of 64-k stages through registers, several blocks per CU: many outputs of
+//                  a short K, and N or K of 2^24 and more.
 //   k_gemm_skinny  M <= 16 rows (speculative-verify shapes): HBM-bound on B.  Split-K, B streamed
 //   (_mfma)        once through LDS, int32 atomics into C (exact and order independent).
 //   k_gemm_generic byte loads and scalar products: operands under 16 bytes, unaligned rows of 2^24 and more.
@@ -22,10 +23,14 @@ namespace {
 // Tile order: blocks are dealt to the 8 XCDs round-robin, so block b runs on XCD b%8.  Give each
 // XCD a contiguous range of tile ids, and walk tile ids in groups of GROUP_M tile rows so the
 // tiles of one XCD share A row panels and B column panels in its L2.
+// EVEN: only where the ids divide evenly, else block order (k_gemm_mfma: C of few rows is written at a
+// higher rate in that order, 256 x 278640 x 144 107 -> 90 us).
+template <bool EVEN = false>
 X100_DEV void tile_coords(int bid, int nblk, int tiles_m, int tiles_n, int &tm, int &tn)
 {
     const int x = bid & 7, q = nblk >> 3;
-    const int t = x * q + min(x, nblk & 7) + (bid >> 3);
+    int t = x * q + min(x, nblk & 7) + (bid >> 3);
+    if (EVEN && (nblk & 7)) t = bid;
     constexpr int GROUP_M = 4;
     int per_group = GROUP_M * tiles_n;
     int g = t / per_group;
@@ -38,8 +43,10 @@ X100_DEV void tile_coords(int bid, int nblk, int tiles_m, int tiles_n, int &tm, 
 
 // ------------------------------------------------------------------------------------------------
 // k_gemm_mfma: tiles of 64-k stages through registers into two LDS buffers (A in 16-byte chunks, B
-// transposed in registers into dwords of four consecutive k of one column).  Offsets are 64-bit and an
-// index past the end is compared as unsigned: any M, N and K of aligned operands.
+// transposed in registers into dwords of four consecutive k of one column).  Two (128x128) to five blocks
+// per CU, so that one block's C traffic, start and end run under the others' products: the faster kernel
+// where C's bytes outweigh the stages (mfma_better in gemm_plan.h has the line and both sides' times).
+// Offsets are 64-bit and an index past the end is compared as unsigned: any M, N and K of aligned operands.
 // ------------------------------------------------------------------------------------------------
 constexpr int BK = 64;   // k bytes per stage
 
@@ -69,7 +76,7 @@ __global__ __launch_bounds__(WM *WN * 64) void k_gemm_mfma(int M, int N, int K,
     const int wm = wave / WN, wn = wave % WN;
     const int lcol = lane & 31, lgrp = lane >> 5;
     int tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+    tile_coords<true>(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     // EDGE = false is only launched when M % BM == 0, N % BN == 0 and K % BK == 0.
     const bool full_mn = !EDGE || (M - m0 >= BM && N - n0 >= BN);
@@ -668,8 +675,8 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_big(int M, int N, int K, const
 //   64 x 64 tiles: 17.5 us with fragments read and used in the same stage, 13.1, 11.9, 10.7).
 // * C is read (ACC) first and written as dwords (32 lanes = one 128-byte row segment): any alignment.
 // Bound by operand delivery (L2 to LDS, 12-16 TB/s over the chip) with many tiles and by the stage's
-// latency with few.  In place of k_gemm_mfma's tiles and of scalar products on unaligned
-// shapes: 333 x 6144 x 2048 26.7 -> 11.7 us, 2048^3 24.3 -> 15.0, 1001 x 1503 x 999 178 -> 10.3.
+// latency with few.  In place of k_gemm_mfma's tiles (which keep the products of a short K) and
+// of scalar products on unaligned shapes: 333 x 6144 x 2048 26.7 -> 11.7 us, 2048^3 24.3 -> 15.0, 1001 x 1503 x 999 178 -> 10.3.
 // ------------------------------------------------------------------------------------------------
 typedef int v4i_u __attribute__((ext_vector_type(4), aligned(1)));
 

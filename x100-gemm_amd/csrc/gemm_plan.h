@@ -2,6 +2,8 @@
 // that a test can evaluate it, with the kernels' 32-bit offsets, at sizes that no test multiplies.
 #pragma once
 #include <math.h>
+
+#include <algorithm>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -35,10 +37,12 @@ inline double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
     struct Cost {
         int bm, bn;
         double start, lat, thr;   // thr: a stage of 256 tiles
+        int res;                  // blocks resident at once (LDS)
+        double round;             // each further round of them: their start and C are not hidden
     };
     static const Cost costs[2][NTILE] = {
-        {{64, 128, 3.6, 0.60, 0.85}, {64, 64, 3.3, 0.38, 0.46}, {32, 64, 2.95, 0.33, 0.36}, {32, 32, 2.7, 0.25, 0.30}},
-        {{128, 128, 3.9, 0.35, 0.60}, {64, 64, 3.1, 0.12, 0.245}, {32, 64, 2.95, 0.10, 0.172}, {32, 32, 2.65, 0.095, 0.155}}};
+        {{64, 128, 3.6, 0.60, 0.85, 256, 0}, {64, 64, 3.3, 0.38, 0.46, 256, 0}, {32, 64, 2.95, 0.33, 0.36, 256, 0}, {32, 32, 2.7, 0.25, 0.30, 256, 0}},
+        {{128, 128, 3.9, 0.35, 0.60, 256, 1.5}, {64, 64, 3.1, 0.12, 0.245, 512, 0.8}, {32, 64, 2.95, 0.10, 0.172, 768, 0.3}, {32, 32, 2.65, 0.095, 0.155, 1280, 0}}};
     const Cost &c = costs[aln][t];
     const double tiles = (double)((M - 1) / c.bm + 1) * ((N - 1) / c.bn + 1), stages = (K - 1) / 128 + 1;
     double per;
@@ -48,7 +52,7 @@ inline double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
     } else {
         per = fmax(c.lat, tiles / 256 * c.thr);
     }
-    return c.start + c_us(M, N, acc) + per * stages;
+    return c.start + c_us(M, N, acc) + per * stages + (ceil(tiles / c.res) - 1) * c.round;
 }
 inline Tile best_tile(bool aln, int M, int N, int K, bool acc, double &us)
 {
@@ -99,13 +103,37 @@ inline bool big_fits(int M, int N, int K, bool acc)
 }
 
 // k_gemm_mfma's tile by output size.  1024^2 x 4096 took 27.3 us on 64x64 tiles and 39.9 on 128x128, 2048^2 x
-// 4096 52.6 on 128x128; 256^3 3.5 on 32x32 and 5.7 on 128x128.
-inline Tile mfma_tile(int M, int N)
+// 4096 52.6 on 128x128; 256^3 3.5 on 32x32 and 5.7 on 128x128.  Up to 64 rows or columns a 128x128 tile is half
+// empty, which a short K shows (27 x 521408 x 64 50 against 31).
+inline bool tile_launches(Tile t, bool aln, int M, int N);
+inline Tile mfma_tile(int M, int N, int K)
 {
     const double mn = (double)M * N;
+    if (std::min(M, N) <= 64 && K <= 128 && mn >= 1e6 && tile_launches(T64, true, M, N)) return T64;
     return mn >= 4.0 * 1024 * 1024 ? T128 : mn >= 1024.0 * 1024 ? T64 : T32;
 }
-
+// Where k_gemm_mfma is the faster one: many outputs of a short K.  C's bytes are most of the time there, and
+// two to five of its blocks share a CU, so that one block's C, start and end run under the others' products;
+// T128 of k_gemm_tile has the CU for itself and T64 half of it.  us, k_gemm_mfma / k_gemm_tile:
+//   C = A.B    256x416544x16   85 / 119    4096x4096x64   14.2 / 17.6    1024^2 x 64    3.6 / 4.2
+//              16384^2 x 256  225 / 318    4096x4096x256  17.9 / 19.4    768x2944x192   5.2 / 6.7
+//              256x2^20x256   307 / 425    1299x30864x368 66 / 55        9476x11984x512 190 / 169
+//   C += A.B   4096x4096x64    22 / 34     4096x4096x256  27.3 / 38.6    7168x4096x320  50 / 60
+//              50769x64x64    6.0 / 8.1    35584x192x128  18.8 / 12.6    31x209280x128  28 / 15
+// The line is fitted to 2146 seeded sizes with K up to 1024 timed on both, a size that k_gemm_mfma would slow
+// down counting twice.  It lies furthest where M, N and K divide into whole tiles and stages (no guards); C +=
+// A.B, whose C k_gemm_tile reads under its stages, leaves the guarded form less, and so do 64x64 tiles and up to
+// 64 rows or columns, where A or B is most of the traffic.
+inline bool mfma_better(int M, int N, int K, bool acc)
+{
+    const double mn = 1e-6 * M * N;   // million outputs
+    if (M <= 16 || mn < 1.0 || K > 448) return false;
+    const int b = mfma_tile(M, N, K) == T128 ? 128 : 64;
+    if (std::min(M, N) <= 64) return K <= (acc ? 64.0 : std::min(192.0, 96 * pow(mn, 0.15)));
+    if (M % b == 0 && N % b == 0 && K % 64 == 0) return K <= (b == 128 ? std::min(448.0, 176 * pow(mn, 0.45)) : std::min(320.0, 224 * pow(mn, 0.45)));
+    if (b == 64) return mn >= 1.5 && K <= std::min(208.0, 160 * pow(mn, 0.30));
+    return K <= (acc ? std::min(224.0, 64 * pow(mn, 0.30)) : std::min(448.0, 112 * pow(mn, 0.30)));
+}
 // Threads of a launch of k_gemm_tile: the runtime takes at most 2^32 - 1 (one column of tiles reaches that at
 // M = 2^30, where k_gemm_mfma's 128x128 tiles, 256 threads each, and the generic kernel's grid do not).
 inline bool tile_launches(Tile t, bool aln, int M, int N)
@@ -140,10 +168,11 @@ inline GemmPlan gemm_plan(int M, int N, int K, bool aligned, bool acc, int varia
         double us = 0;
         if (aligned && skinny && (!tiled || skinny_us(M, N, K, acc) <= skinny_tile_us(t, M, N, K, acc)))
             return {GK_SKINNY, t, true};
-        if (!tiled) return aligned && whole ? GemmPlan{GK_BIG8, t, true} : on_tile(mfma_tile(M, N));
+        if (!tiled) return aligned && whole ? GemmPlan{GK_BIG8, t, true} : on_tile(mfma_tile(M, N, K));
+        if (aligned && !whole && mfma_better(M, N, K, acc)) return {GK_MFMA, mfma_tile(M, N, K), true};
         t = best_tile(aligned, M, N, K, acc, us);
         if (aligned && whole && us >= big_us(M, N, K, acc)) return {GK_BIG8, t, true};
-        return on_tile(tile_launches(t, aligned, M, N) ? t : mfma_tile(M, N));
+        return on_tile(tile_launches(t, aligned, M, N) ? t : mfma_tile(M, N, K));
     }
     case X100_GEMM_TILE256: return whole ? GemmPlan{GK_BIG8, T128, true} : on_tile(T128);
     case X100_GEMM_TILE256_W4: return whole ? GemmPlan{GK_BIG4, T128, true} : on_tile(T128);

@@ -65,3 +65,31 @@ def test_tile(dev, int4, N, K, M):
     got = dy.cpu().numpy()
     assert (got[M * N:] == -7).all()
     assert np.array_equal(got[:M * N].reshape(M, N), ol.gemv_int(W, x))
+
+
+@pytest.mark.parametrize("int4,K", [(False, 16), (False, 32), (True, 32)])
+def test_tile_2_28_rows(dev, int4, K):
+    # one launch of four waves per 16 rows would pass 2^32 - 1 threads; the first, last and some other rows
+    import torch
+    M, N = 2, 1 << 28
+    g = torch.Generator(device=dev).manual_seed(K)
+    nb = N * K // (2 if int4 else 1)
+    W = torch.randint(0, 256, (nb,), generator=g, device=dev, dtype=torch.uint8)
+    x = synth.rand_int8(K, (M, K))
+    dx = torch.from_numpy(x).to(dev)
+    dy = torch.full((M * N + 64,), -7, dtype=torch.int32, device=dev)
+    x100hip.gemv_tile(int4, M, N, K, W.data_ptr(), dx.data_ptr(), dy.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert (dy[M * N:] == -7).all()
+    blocks = np.unique(np.concatenate([np.arange(16), N // 8 - 16 + np.arange(16), np.random.default_rng(K).integers(0, N // 8, 500)]))
+    tiles = W.reshape(N // 8, -1, 8, 16)[torch.from_numpy(blocks).to(dev)].cpu().numpy()   # [block][tile][row][16 bytes]
+    got = dy[:M * N].reshape(M, N // 8, 8)[:, torch.from_numpy(blocks).to(dev)].cpu().numpy()
+    del W, dy
+    torch.cuda.empty_cache()
+    if int4:
+        lo, hi = (tiles << 4).view(np.int8) >> 4, tiles.view(np.int8) >> 4
+        rows = np.concatenate([lo, hi], axis=3)
+    else:
+        rows = tiles.view(np.int8)
+    rows = rows.transpose(0, 2, 1, 3).reshape(len(blocks), 8, K).astype(np.int64)
+    assert np.array_equal(got, np.einsum("mk,bnk->mbn", x.astype(np.int64), rows))

@@ -299,7 +299,9 @@ hipError_t launch_tile(bool int4, int M, int N, int K, const void *W, const int8
 }
 
 // k_gemv_tile_mm with S waves per 16 rows and U steps per pass (4 waves on K unless the rows alone fill
-// the chip and K is short; int8 from K = 1024 up with 8 steps in flight per wave).
+// the chip and K is short; int8 from K = 1024 up with 8 steps in flight per wave).  S = 4 takes 16 threads
+// per row, which passes the 2^32 - 1 of one launch at N = 2^28: two waves from there (up to 2^29, as
+// k_gemv_tile).
 hipError_t launch_tile_mm(bool int4, int M, int N, int K, const void *W, const int8_t *x, int32_t *y, hipStream_t s)
 {
     const int steps = ((int4 ? K / 32 : K / 16) + 3) / 4, pitch = (K + 255) / 256 * 256 + 16;
@@ -307,12 +309,14 @@ hipError_t launch_tile_mm(bool int4, int M, int N, int K, const void *W, const i
         hipLaunchKernelGGL(k, dim3(((N / 8 + 1) / 2 * S + 3) / 4), dim3(256), (size_t)M * pitch + 16, s, M, N, K, pitch,
                            udiv16_magic((uint32_t)(K / 16)), (const uint8_t *)W, x, y);
     };
+    const bool wide = N >= 1 << 28;
     if (int4) {
-        if (N >= 16384 && steps <= 8) go(k_gemv_tile_mm<true, 2, 4>, 2);
+        if (wide || (N >= 16384 && steps <= 8)) go(k_gemv_tile_mm<true, 2, 4>, 2);
         else if (steps <= 8) go(k_gemv_tile_mm<true, 4, 2>, 4);
         else go(k_gemv_tile_mm<true, 4, 4>, 4);
     } else {
-        if (steps <= 8) go(k_gemv_tile_mm<false, 4, 2>, 4);
+        if (wide) go(k_gemv_tile_mm<false, 2, 4>, 2);
+        else if (steps <= 8) go(k_gemv_tile_mm<false, 4, 2>, 4);
         else if (steps <= 16) go(k_gemv_tile_mm<false, 4, 4>, 4);
         else go(k_gemv_tile_mm<false, 4, 8>, 4);
     }

@@ -50,7 +50,10 @@ def test_q4_0(dev, N, K, M):
 
 @pytest.mark.parametrize("int4", [True, False])
 @pytest.mark.parametrize("N,K,M", [(8, 32, 2), (24, 160, 3), (16, 992, 5), (1000, 1056, 8), (1024, 2080, 2), (264, 4864, 8),
-                                   (16384, 1024, 4), (65536, 1024, 1), (40, 6528, 7), (2056, 96, 6)])
+                                   (16384, 1024, 4), (65536, 1024, 1), (40, 6528, 7), (2056, 96, 6),
+                                   # fewer waves per 16 rows: 16384 and 65536 rows, K to 8 steps, last block part full
+                                   (16384, 32, 2), (16392, 480, 5), (65528, 512, 8), (65536, 64, 3), (65544, 544, 2),
+                                   (65544, 992, 8), (80008, 160, 7)])
 def test_tile(dev, int4, N, K, M):
     import torch
     W = synth.rand_int8(N + K, (N, K))

@@ -298,10 +298,12 @@ hipError_t launch_tile(bool int4, int M, int N, int K, const void *W, const int8
     }
 }
 
-// k_gemv_tile_mm with S waves per 16 rows and U steps per pass (4 waves on K unless the rows alone fill
-// the chip and K is short; int8 from K = 1024 up with 8 steps in flight per wave).  S = 4 takes 16 threads
-// per row, which passes the 2^32 - 1 of one launch at N = 2^28: two waves from there (up to 2^29, as
-// k_gemv_tile).
+// k_gemv_tile_mm with S waves per 16 rows and U steps per pass: four waves on K (int8 from K = 1024 up with 8
+// steps in flight per wave), fewer where the rows fill the chip and K is at most eight steps, which four waves
+// cut to two or less each.  us, M = 2 and 8, dot products / S = 4 / 2 / 1: int8 131072x128 5.9, 8.5 / 8.0, 8.3 /
+// 6.1, 6.6 / 3.7, 4.1; 40960x256 3.4, 5.0 / 4.1, 4.2 / 3.5, 3.6 / 3.5, 3.6; 65536x512 4.5, 8.1 / 5.2, 5.5 / 4.2,
+// 4.4 / 4.2, 4.5; int4 65536x256 4.1, 6.7 / - / 4.9, 4.8 / 3.7, 3.6.  S = 4 takes 16 threads per row, which passes
+// the 2^32 - 1 of one launch at N = 2^28.
 hipError_t launch_tile_mm(bool int4, int M, int N, int K, const void *W, const int8_t *x, int32_t *y, hipStream_t s)
 {
     const int steps = ((int4 ? K / 32 : K / 16) + 3) / 4, pitch = (K + 255) / 256 * 256 + 16;
@@ -309,13 +311,15 @@ hipError_t launch_tile_mm(bool int4, int M, int N, int K, const void *W, const i
         hipLaunchKernelGGL(k, dim3(((N / 8 + 1) / 2 * S + 3) / 4), dim3(256), (size_t)M * pitch + 16, s, M, N, K, pitch,
                            udiv16_magic((uint32_t)(K / 16)), (const uint8_t *)W, x, y);
     };
-    const bool wide = N >= 1 << 28;
+    const bool rows = steps <= 8 || N >= 1 << 28;   // enough of them: fewer waves per 16
     if (int4) {
-        if (wide || (N >= 16384 && steps <= 8)) go(k_gemv_tile_mm<true, 2, 4>, 2);
+        if (rows && N >= 65536) go(k_gemv_tile_mm<true, 1, 2>, 1);
+        else if (rows && N >= 16384) go(k_gemv_tile_mm<true, 2, 4>, 2);
         else if (steps <= 8) go(k_gemv_tile_mm<true, 4, 2>, 4);
         else go(k_gemv_tile_mm<true, 4, 4>, 4);
     } else {
-        if (wide) go(k_gemv_tile_mm<false, 2, 4>, 2);
+        if (rows && N >= 65536) go(k_gemv_tile_mm<false, 1, 2>, 1);
+        else if (rows && N >= 16384) go(k_gemv_tile_mm<false, 2, 4>, 2);
         else if (steps <= 8) go(k_gemv_tile_mm<false, 4, 2>, 4);
         else if (steps <= 16) go(k_gemv_tile_mm<false, 4, 4>, 4);
         else go(k_gemv_tile_mm<false, 4, 8>, 4);
@@ -323,15 +327,17 @@ hipError_t launch_tile_mm(bool int4, int M, int N, int K, const void *W, const i
     return hipGetLastError();
 }
 
-// The matrix cores take several token rows; one row where the launch streams enough weights (us, dot
-// products / matrix cores; int4, int8): 151936x2048 M = 1 27.6 / 25.6, 47.5 / 44.5, M = 2 29.0 / 26.2,
-// M = 8 54.7 / 29.3, 60.6 / 48.3; 4864x896 M = 1 2.8 / 2.8, 3.2 / 3.2, M = 8 5.0 / 2.9, 5.3 / 3.2.  With
-// few rows and a long K, 2 or 3 rows stay on the dot products (256x4864 int8 M = 3 4.8 / 4.4, M = 2
-// 4.4 / 4.4; int4 3.6 / 3.7): too few 16-row tiles to split K over.
-inline bool tile_mm(bool int4, int M, int N, int K)
+// The matrix cores take three token rows and more; one row where the launch streams enough weights, two rows
+// in between (us, dot products / matrix cores; int4, int8): 151936x2048 M = 1 27.6 / 25.6, 47.5 / 44.5, M = 8
+// 54.7 / 29.3, 60.6 / 48.3; 4864x896 M = 1 2.8 / 2.8, 3.2 / 3.2, M = 8 5.0 / 2.9, 5.3 / 3.2.  With two rows the
+// dot products keep a short K (30304x32 int4 3.4 / 3.7; 14536x160 int8 2.9 / 3.1) until 65536 rows, and a long K
+// with too few 16-row tiles to split it over (1256x9216 int4 4.5 / 5.6).
+inline bool tile_mm(int M, int N, int K)
 {
-    if (M == 1) return N >= 65536 && K >= 1024;
-    return M > 2 || N >= 1024 || K <= 2048 || !int4;
+    if (M > 2) return true;
+    if (N >= 65536) return M == 2 || K >= 1024;
+    if (M == 1) return false;
+    return K <= 512 ? K > 128 && N < 4096 : K <= 2048 || N >= 4096;
 }
 
 }  // namespace
@@ -341,7 +347,7 @@ hipError_t x100_gemv_tile_launch(int int4, int M, int N, int K, const void *W, c
 {
     if (M < 1 || M > 8 || N < 8 || N % 8 || K < 16 || K % (int4 ? 32 : 16)) return hipErrorInvalidValue;
     if ((size_t)M * K + 16 + ((size_t)M * (K / 16) + 1) * 4 > 64 * 1024) return hipErrorInvalidValue;
-    if (tile_mm(int4 != 0, M, N, K)) return launch_tile_mm(int4 != 0, M, N, K, W, x, y, s);
+    if (tile_mm(M, N, K)) return launch_tile_mm(int4 != 0, M, N, K, W, x, y, s);
     if (M == 1) return launch_tile<1>(int4 != 0, M, N, K, W, x, y, s);
     return launch_tile<2>(int4 != 0, M, N, K, W, x, y, s);   // M = 2
 }

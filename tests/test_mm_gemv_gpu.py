@@ -53,7 +53,9 @@ def test_q4_0(dev, N, K, M):
                                    (16384, 1024, 4), (65536, 1024, 1), (40, 6528, 7), (2056, 96, 6),
                                    # fewer waves per 16 rows: 16384 and 65536 rows, K to 8 steps, last block part full
                                    (16384, 32, 2), (16392, 480, 5), (65528, 512, 8), (65536, 64, 3), (65544, 544, 2),
-                                   (65544, 992, 8), (80008, 160, 7)])
+                                   (65544, 992, 8), (80008, 160, 7),
+                                   # two rows: both sides of the lines to the dot products
+                                   (4088, 160, 2), (4096, 512, 2), (65528, 480, 2), (65536, 480, 2), (4088, 2080, 2), (4096, 2080, 2)])
 def test_tile(dev, int4, N, K, M):
     import torch
     W = synth.rand_int8(N + K, (N, K))

@@ -14,7 +14,10 @@ pytestmark = pytest.mark.gpu
 # N below, at and past the 16- and 32-row tiles and the 4096 / 8192 / 16384-row plan changes
 I8 = [(16, 512, 2), (17, 480, 8), (33, 32, 3), (100, 544, 3), (31, 1024, 5), (48, 992, 8), (512, 2048, 5), (8200, 2048, 8),
       (15, 1056, 6), (777, 2016, 8), (2048, 4096, 5), (130, 2080, 8), (65, 3968, 7), (129, 8192, 7), (40, 4128, 8),
-      (1, 2048, 8)]
+      (1, 2048, 8),
+      # K <= 1024 and few rows of x: both sides of the lines by N
+      (8191, 96, 2), (8192, 512, 2), (12287, 32, 3), (12288, 480, 3), (114689, 64, 3), (24575, 128, 4), (24576, 256, 4),
+      (57345, 32, 4), (2047, 1024, 3), (2048, 992, 4), (81921, 544, 4)]
 Q4 = [(16, 512, 5), (512, 2048, 8), (4099, 2048, 5), (8193, 1024, 2), (31, 1984, 7), (1, 32, 8), (129, 4096, 8),
       (8200, 2080, 3), (16390, 4096, 2), (33, 3968, 6), (17, 8192, 2), (130, 4128, 4), (48, 8160, 8)]
 

@@ -1397,8 +1397,9 @@ hipError_t launch_q_mm(int M, int N, int K, const void *w, const float *x, float
 // Where the matrix cores win (us, k_q_mm against the dot-product kernels, M = 8 unless said; LPR and BPL
 // as those kernels take them from K).  The plans spread x's quantization over 512 or 1024 threads;
 // with few rows of x the dot products cost less than that spread's fixed steps.
-//   int8  K <= 512, M >= 2 (777x480: M = 2 2.7 / 3.2, M = 8 2.9 / 5.2)
-//         K <= 1024, M >= 3 (4096x1024: M = 3 3.5 / 3.8, M = 8 3.8 / 5.4)
+//   int8  K <= 512, M >= 5, and fewer rows where few or very many weight rows leave the persistent grid whole
+//         rounds (777x480: M = 2 2.7 / 3.2, M = 8 2.9 / 5.2; 26112x448: M = 2 4.8 / 3.9; 27754x416: M = 4 5.3 / 4.6)
+//         K <= 1024 likewise (1280x1024: M = 4 3.3 / 3.8; 12947x768: M = 3 5.5 / 4.3; 90797x832: M = 4 14.9 / 16.4)
 //         K <= 4096, M >= 5 (4096x2048 5.1 / 6.7, M = 4 4.6 / 4.5; 151936x2048 68 / 80, M = 4 65 / 61;
 //                            8192x4096 11.8 / 15.8)
 //         K <= 8192, M >= 7 (4099x8000 16.8 / 20.2, 2048x8192 14.3 / 14.6, M = 5 13.1 / 11.8)
@@ -1419,8 +1420,13 @@ hipError_t launch_mm(bool q4, int M, int N, int K, const void *w, const float *x
         return N >= 4096 ? launch_q_mm<true, 8, 1, 8, 2, 4>(M, N, K, w, x, y, s)
                          : launch_q_mm<true, 4, 1, 16, 1, 4>(M, N, K, w, x, y, s);
     }
-    if (nb <= 16) return launch_q_mm<false, 4, 1, 4, 1, 4>(M, N, K, w, x, y, s);
-    if (nb <= 32) return M >= 3 ? launch_q_mm<false, 4, 2, 4, 1, 8>(M, N, K, w, x, y, s) : hipErrorNotSupported;
+    if (nb <= 16) {
+        const bool few = N < (M == 2 ? 8192 : M == 3 ? 12288 : 24576), many = M > 2 && N >= (M == 3 ? 114688 : 57344);
+        return M >= 5 || few || many ? launch_q_mm<false, 4, 1, 4, 1, 4>(M, N, K, w, x, y, s) : hipErrorNotSupported;
+    }
+    if (nb <= 32)
+        return M >= 5 || (M >= 3 && (N < 2048 || N >= 81920)) ? launch_q_mm<false, 4, 2, 4, 1, 8>(M, N, K, w, x, y, s)
+                                                              : hipErrorNotSupported;
     if (M < (nb <= 128 ? 5 : 7)) return hipErrorNotSupported;
     if (nb <= 64)
         return N >= 8192 ? launch_q_mm<false, 2, 4, 8, 2, 4>(M, N, K, w, x, y, s)

@@ -1509,7 +1509,16 @@ hipError_t moe_launch_mfma(int M, int d, int ff, int n_exp, int n_act, const flo
 {
     const int nsb = d / 256, nsf = ff / 256, P = M * n_act, nrc = (M + 7) / 8;
     const int Vmax = min(P, (P + MF_PCH - 1) / MF_PCH + n_exp), Vr = (Vmax + 7) & ~7;   // chunks at most
-    const int vr = P >= 24 * n_exp ? 0 : Vmax;   // block order (k_moe_mfma)
+    // Block order (k_moe_mfma).  us, plain / by XCD, d = 2048, ff = 768 unless said, n_act 8 (4 experts: 1):
+    //   pairs per expert            6            12           16           24           32           48           64
+    //   128 experts            103 / 107    115 / 116    134 / 134    149 / 141    193 / 188
+    //   60 experts              59 / 58      65 / 63      68 / 68      80 / 75      98 / 96     126 / 118    147 / 135
+    //   32 experts              49 / 47      51 / 49      53 / 51      66 / 60      65 / 65      75 / 70      89 / 85
+    //   4 experts                                         41 / 41                   45 / 44
+    // from 24 on no worse than level with 8 experts and more, below it either may be ahead (64 experts, 16: 65 /
+    // 69; d = 4096, ff = 1024, 16 experts, 12: 69 / 58).  Fewer chunks than XCDs leave XCDs idle: one expert, 32
+    // rows, ff = 3072 47.5 / 54.9; 4 experts, 512 rows 53 / 58.
+    const int vr = n_exp >= 8 && P >= 24 * n_exp ? 0 : Vmax;
     const int nc = vr ? Vmax : Vr;
     route_rows(M, d, n_exp, hn, R, ws, s);
     hipLaunchKernelGGL(k_moe_topk_rows, dim3(nrc), dim3(512), 0, s, M, n_exp, n_act, ws, sel, sw);

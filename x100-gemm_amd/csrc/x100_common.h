@@ -11,6 +11,8 @@
 
 #include <type_traits>
 
+#include "resident_cache.h"
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
@@ -543,30 +545,20 @@ X100_DEV float q4k_term(float d, float dmin, float dx, int isc, int imn)
 
 // Blocks of kernel k that are resident on the whole device at once with lds bytes of dynamic LDS
 // (the runtime's occupancy for the kernel times the CU count): the grid of a persistent launch.
-// Cached per calling thread, keyed by (kernel address, block size, device, lds): template
-// instances with the same signature are distinct kernels with distinct occupancy.
-struct ResidentKey {
-    const void *k;
-    int nt, dev;
-    size_t lds;
-    int blocks;
-};
+inline int resident_blocks_of(const void *k, int nt, size_t lds)
+{
+    static thread_local ResidentCache cache;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+    return cache.get({k, nt, dev, lds}, [&] {
+        int occ = 0, cus = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, nt, lds) != hipSuccess || occ < 1) occ = 1;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+        return occ * cus;
+    });
+}
 template <typename Kern>
 inline int resident_blocks(Kern k, int nt, size_t lds)
 {
-    static thread_local ResidentKey cache[16];
-    static thread_local int used = 0, next = 0;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    const void *kp = (const void *)k;
-    for (int i = 0; i < used; i++)
-        if (cache[i].k == kp && cache[i].nt == nt && cache[i].dev == dev && cache[i].lds == lds)
-            return cache[i].blocks;
-    int occ = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k, nt, lds) != hipSuccess || occ < 1) occ = 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-        cus = 256;
-    ResidentKey &e = cache[used < 16 ? used++ : (next++ & 15)];
-    e = ResidentKey{kp, nt, dev, lds, occ * cus};
-    return e.blocks;
+    return resident_blocks_of((const void *)k, nt, lds);
 }

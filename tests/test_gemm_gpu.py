@@ -43,8 +43,8 @@ def test_gemm_256_cube(dev):
 
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (8, 4096, 4096), (300, 200, 96), (2048, 2048, 1024)])
 def test_gemm_overwrite_form(dev, M, N, K):
-    # C = A*B whatever C held before (the overwrite form of gemm_ime2_i8_st / _mt): the MFMA tiles,
-    # the skinny split-K kernel (atomics into the cleared C) and the generic kernel.
+    # C = A*B whatever C held before (the overwrite form of gemm_ime2_i8_st / _mt): the MFMA tiles
+    # and the skinny split-K kernel (atomics into the cleared C).
     import torch
     A, B = synth.gemm_inputs(M, N, K, seed=3030 + M)
     garbage = synth.rand_int8(5, (M, N)).astype(np.int32) * 12345
@@ -57,7 +57,7 @@ def test_gemm_overwrite_form(dev, M, N, K):
 
 
 # (variant, M, N, K): every kernel's overwrite form.  The 256x256 kernel with superstages (K / 64 a
-# multiple of 8) and without (K = 576), 8 and 4 waves; the register-staged tiles with and without
+# multiple of 8) and without (K = 576), 8 and 4 waves; k_gemm_tile's tiles with and without
 # edges; the generic kernel; the skinny split-K kernels (cleared C + atomics).
 SET_CASES = [(x100hip.GEMM_TILE256, 4096, 4096, 4096), (x100hip.GEMM_TILE256, 512, 768, 576),
              (x100hip.GEMM_TILE256_W4, 1024, 512, 1024), (x100hip.GEMM_TILE256_W4, 256, 512, 576),
@@ -183,10 +183,12 @@ def test_gemm_forced_variants(dev, variant, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(5, 20, 40), (64, 30, 64), (9, 17, 33), (100, 100, 100)])
 def test_gemm_unaligned_shapes(dev, M, N, K):
-    # K or N not a multiple of 16: row starts are not 16-byte aligned -> generic kernel
+    # K or N not a multiple of 16: row starts are not 16-byte aligned -> k_gemm_tile's unaligned form, and the
+    # generic kernel on request
     A, B = synth.gemm_inputs(M, N, K, seed=M + N + K)
     C0 = np.zeros((M, N), np.int32)
     assert np.array_equal(gpu_gemm(A, B, C0, dev), oracle_gemm(A, B, C0))
+    assert np.array_equal(gpu_gemm(A, B, C0, dev, x100hip.GEMM_GENERIC), oracle_gemm(A, B, C0))
 
 
 def test_gemm_extremes(dev):
@@ -226,8 +228,8 @@ def test_gemm_host_dropin_reuses_buffers(dev):
     # one (the buffers grow), a smaller one again (the larger buffers hold stale data beyond it),
     # and two host threads at once (calls on one device run one at a time).
     import threading
-    # (2048, 1280, 1024): C is 10 MiB, two 8 MiB staging chunks, the second partial; A and B share
-    # the chunk stream with C
+    # (2048, 1280, 1024): A.B is 10 MiB, three 4 MiB staging chunks, the last partial (inputs of more chunks
+    # than slots: test_gemm_host_add_gpu.py)
     for i, (M, N, K) in enumerate([(40, 48, 32), (512, 384, 256), (24, 16, 48), (256, 272, 1040),
                                    (2048, 1280, 1024), (64, 48, 16)]):
         A, B = synth.gemm_inputs(M, N, K, seed=60 + i)

@@ -80,3 +80,10 @@ def test_short_k_takes_the_kernel_with_several_blocks_per_cu(plans):
     fast = [(333, 6144, 2048, 0), (256, 256, 256, 1), (2000, 8128, 512, 1), (512, 512, 64, 0), (31, 209280, 128, 1),
             (35584, 192, 128, 1), (1024, 3584, 384, 0)]
     assert {p[0] for p in plans([(M, N, K, 1, acc, 0) for M, N, K, acc in fast])} == {"tile"}
+
+
+def test_the_gpu_tests_reach_every_form_of_the_tiles(plans):
+    from test_gemm_tile_gpu import FORMS
+    cases = [(M, N, K, a, acc, 0) for _, a, M, N, K in FORMS for acc in (0, 1)]
+    want = [("tile", t, a) for t, a, *_ in FORMS for _ in (0, 1)]
+    assert [p[:3] for p in plans(cases)] == want

@@ -63,3 +63,19 @@ def test_tile_base_address(dev, M, N, K, off):
 def test_tile_auto(dev, M, N, K):
     run(dev, M, N, K, True)
     run(dev, M, N, K, False)
+
+
+# Every form of the automatic choice over its pipeline: (tile, aligned, M, N, K).  The aligned 32x64 tile, which no
+# variant selects, over the ring's unrolled turn (8 stages and more) and K tails; the unaligned tiles over two to
+# twenty stages.  test_gemm_plan.py checks that the sizes take these tiles.
+FORMS = [("32x64", 1, 97, 3088, 272), ("32x64", 1, 130, 2064, 1040), ("32x64", 1, 97, 2064, 1168), ("32x64", 1, 180, 1040, 2096),
+         ("128", 0, 1001, 1503, 999), ("128", 0, 1300, 1503, 514), ("128", 0, 700, 2049, 1155), ("128", 0, 2047, 1601, 385),
+         ("64", 0, 1100, 1300, 257), ("64", 0, 2049, 1153, 515), ("64", 0, 1025, 1600, 270),
+         ("32x64", 0, 700, 777, 131), ("32x64", 0, 700, 777, 387), ("32x64", 0, 700, 777, 514), ("32x64", 0, 513, 771, 1023),
+         ("32", 0, 37, 41, 2500), ("32", 0, 300, 300, 1201)]
+
+
+@pytest.mark.parametrize("tile,aligned,M,N,K", FORMS)
+def test_tile_forms(dev, tile, aligned, M, N, K):
+    run(dev, M, N, K, True)
+    run(dev, M, N, K, False)

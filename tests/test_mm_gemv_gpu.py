@@ -51,6 +51,29 @@ def test_q4_0(dev, N, K, M):
     check(dev, synth.Q4_0, N, K, M)
 
 
+def test_q4_0_past_2_27_blocks(dev):
+    # 2^20 + 3 rows of 128 blocks: the dot-product kernel's 64-bit offsets; sampled rows against the oracle
+    import torch
+    M, N, K = 5, (1 << 20) + 3, 4096
+    s = torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(1)
+    raw = torch.randint(0, 256, (N, K // 32, 18), generator=g, device=dev, dtype=torch.uint8)
+    raw[..., 1] = 0x18                 # fp16 scales of about 0.002
+    packed = torch.empty(x100hip.packed_bytes(synth.Q4_0, N, K), dtype=torch.uint8, device=dev)
+    x100hip.pack(synth.Q4_0, N, K, raw.data_ptr(), packed.data_ptr(), s)
+    x = synth.normal_f32(2, (M, K))
+    dx, dy = torch.from_numpy(x).to(dev), torch.empty((M, N), dtype=torch.float32, device=dev)
+    x100hip.qgemv(synth.Q4_0, M, N, K, packed.data_ptr(), dx.data_ptr(), dy.data_ptr(), s)
+    torch.cuda.synchronize()
+    rows = np.concatenate([np.arange(8), np.random.default_rng(3).integers(0, N, 100), np.arange(N - 8, N)])
+    at = torch.from_numpy(rows).to(dev)
+    W, got = raw[at].cpu().numpy(), dy[:, at].cpu().numpy()
+    del raw, packed, dy
+    torch.cuda.empty_cache()
+    ref = ol.qgemv(synth.Q4_0, np.ascontiguousarray(W), x)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("int4", [True, False])
 @pytest.mark.parametrize("N,K,M", [(8, 32, 2), (24, 160, 3), (16, 992, 5), (1000, 1056, 8), (1024, 2080, 2), (264, 4864, 8),
                                    (16384, 1024, 4), (65536, 1024, 1), (40, 6528, 7), (2056, 96, 6),

@@ -282,8 +282,10 @@ hipError_t launch_tile_s(bool int4, int M, int N, int K, const void *W, const in
     const size_t lds = (size_t)M * K + 16 + ((size_t)M * (K / 16) + 1) * 4;
     if (int4)
         hipLaunchKernelGGL((k_gemv_tile<MR, true, S>), grid, dim3(256), lds, s, M, N, K, (const uint8_t *)W, x, y);
-    else
+    else if constexpr (MR == 1 || S != 2)
         hipLaunchKernelGGL((k_gemv_tile<MR, false, S>), grid, dim3(256), lds, s, M, N, K, (const uint8_t *)W, x, y);
+    else   // two int8 rows come here with K <= 512 (S = 1) or above 2048 (S = 4)
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

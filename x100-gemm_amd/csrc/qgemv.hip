@@ -1368,10 +1368,14 @@ template <int MR>
 hipError_t launch_q8_0(int M, int N, int K, const void *w, const float *x, float *y, hipStream_t s)
 {
     const int nb = K / 32;
-    if (nb <= 16) return launch_q8_0_x<MR, 16, 1>(M, N, K, w, x, y, s);
-    if (nb <= 32) return launch_q8_0_x<MR, 16, 2>(M, N, K, w, x, y, s);
-    if (nb <= 64) return launch_q8_0_x<MR, 16, 4>(M, N, K, w, x, y, s);
-    if (nb <= 128) return launch_q8_0_x<MR, 32, 4>(M, N, K, w, x, y, s);
+    if constexpr (MR <= 4) {
+        if (nb <= 16) return launch_q8_0_x<MR, 16, 1>(M, N, K, w, x, y, s);
+        if (nb <= 32) return launch_q8_0_x<MR, 16, 2>(M, N, K, w, x, y, s);
+        if (nb <= 64) return launch_q8_0_x<MR, 16, 4>(M, N, K, w, x, y, s);
+        if (nb <= 128) return launch_q8_0_x<MR, 32, 4>(M, N, K, w, x, y, s);
+    } else if (nb <= 128) {   // launch_mm takes 5 rows and more of K <= 4096
+        return hipErrorInvalidValue;
+    }
     if (nb <= 256) return launch_q8_0_x<MR, 64, 4>(M, N, K, w, x, y, s);
     return launch_q8_0_x<MR, 64, 8>(M, N, K, w, x, y, s);
 }
@@ -1406,6 +1410,7 @@ hipError_t launch_q_mm(int M, int N, int K, const void *w, const float *x, float
 //   Q4_0  M >= 5 (4096x4096 7.8 / 11.2, 32768x4096 20 / 50), or many rows (16384x2048: M = 2 7.7 / 8.7;
 //         9000x4096: M = 3 10.2 / 10.9, M = 2 9.9 / 9.2; 32768x4096: M = 2 18.6 / 21.5), or K > 4096
 //         (3000x7680: M = 2 8.9 / 9.2, M = 4 10.0 / 11.9)
+// Past 2^27 blocks k_q_mm's 32-bit offsets end: Q4_0 stays on k_q4_0 (the int8 path takes no such weight).
 // hipErrorNotSupported: outside (the caller takes those kernels).
 hipError_t launch_mm(bool q4, int M, int N, int K, const void *w, const float *x, float *y, hipStream_t s)
 {

@@ -87,3 +87,11 @@ def test_the_gpu_tests_reach_every_form_of_the_tiles(plans):
     cases = [(M, N, K, a, acc, 0) for _, a, M, N, K in FORMS for acc in (0, 1)]
     want = [("tile", t, a) for t, a, *_ in FORMS for _ in (0, 1)]
     assert [p[:3] for p in plans(cases)] == want
+
+
+def test_few_rows_of_a_long_k_split_it(plans):
+    # the split-K kernels were up to twice as fast as 32x32 tiles here; and sizes that the tiles win
+    split = [(9, 3072, 9984), (10, 3456, 8768), (16, 3232, 10096), (14, 4096, 13120)]
+    tile = [(16, 1280, 1280), (14, 154960, 80), (14, 174832, 160), (14, 2016, 5792), (12, 2048, 9024)]
+    for sizes, kernel in ((split, "skinny"), (tile, "tile")):
+        assert {p[0] for p in plans([(M, N, K, 1, acc, 0) for M, N, K in sizes for acc in (0, 1)])} == {kernel}, kernel

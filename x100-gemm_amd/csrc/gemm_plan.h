@@ -38,7 +38,7 @@ inline double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
         int bm, bn;
         double start, lat, thr;   // thr: a stage of 256 tiles
         int res;                  // blocks resident at once (LDS)
-        double round;             // each further round of them: their start and C are not hidden
+        double round;             // each further round of them (M > 16): their start and C are not hidden
     };
     static const Cost costs[2][NTILE] = {
         {{64, 128, 3.6, 0.60, 0.85, 256, 0}, {64, 64, 3.3, 0.38, 0.46, 256, 0}, {32, 64, 2.95, 0.33, 0.36, 256, 0}, {32, 32, 2.7, 0.25, 0.30, 256, 0}},
@@ -52,7 +52,7 @@ inline double tile_us(Tile t, bool aln, int M, int N, int K, bool acc)
     } else {
         per = fmax(c.lat, tiles / 256 * c.thr);
     }
-    return c.start + c_us(M, N, acc) + per * stages + (ceil(tiles / c.res) - 1) * c.round;
+    return c.start + c_us(M, N, acc) + per * stages + (M > 16 ? (ceil(tiles / c.res) - 1) * c.round : 0.0);
 }
 inline Tile best_tile(bool aln, int M, int N, int K, bool acc, double &us)
 {
@@ -73,7 +73,8 @@ inline double big_us(int M, int N, int K, bool acc)
 }
 // The split-K kernels for M <= 16 (C = A.B pays a clearing launch).  They stream B at up to 5 TB/s in
 // 128- or 256-column rows; the tiles reach 3.6 TB/s on a B beyond the caches, and less on rows that
-// are not whole cache lines (4x4112x4112: 7.0 us split-K, 9.4 on T32; 16x1280x1280: 7.7 and 3.7).
+// are not whole cache lines (4x4112x4112: 7.0 us split-K, 9.4 on T32; 16x1280x1280: 7.7 and 3.7); few tiles of a
+// long K wait for each stage (9x3072x9984: 10.7 split-K, 22.4 on T32; 10x3456x8768 11.1 and 16.9).
 inline double skinny_us(int M, int N, int K, bool acc)
 {
     const double kn = (double)K * N, clear = acc ? 0.0 : 1.6;
@@ -85,6 +86,7 @@ inline double skinny_tile_us(Tile &t, int M, int N, int K, bool acc)
     double us;
     t = best_tile(true, M, N, K, acc, us);
     if (N % 128) us = 2.65 + 1.5 * (us - 2.65);
+    if ((double)K * N > (N % 128 ? 14e6 : 20e6)) us = fmax(us, 2.65 + 0.205 * ((K - 1) / 128 + 1));   // stages of a B beyond the L2s
     return fmax(us, 2.65 + (double)K * N / 3.6e6);
 }
 

@@ -926,8 +926,9 @@ __global__ __launch_bounds__(256) void k_moe_act_q8k(int P, int ff, MoeWs ws)
 // sum_j m_j S_j (S_j the sum of the activation bytes of sub-block j, S_j = l_j + 64 h_j) takes two
 // v_mfma_i32_32x32x16_i8 per super-block, the m_j against the bytes l_j and h_j that the block packs
 // into LDS once: in place of one full product per sub-block with m_j in every byte (a quarter of the
-// matrix work, and four register copies of each m_j).  Bound by the VALU, whose unpacking and scaling
-// fill it 70% (M = 512).  These integers equal those of the one-row kernels, and the fp32 combine
+// matrix work, and four register copies of each m_j).  At M = 512 the VALU (unpacking,
+// scaling, the fp32 combine) is busy 68% of gate/up and 59% of down, the matrix cores 26% and 25%, and a wave
+// waits to issue a third of its time: none of them alone is the bound.  These integers equal those of the one-row kernels, and the fp32 combine
 // per super-block (q4k_combine) and the sum over super-blocks run in the same order, so every
 // output is bit-identical to theirs.
 //

@@ -4,7 +4,7 @@
 // that falls back to the scalar gemm_ref_i8 (src/gemm_ref.c:17-26).  Integer arithmetic is exact,
 // so every kernel here is bit-identical to gemm_ref_i8 for any K below 2^17 (|sum| < 2^31).
 //
-// Kernels (x100_gemm_i8_launch picks one by sizes and alignment):
+// Kernels (gemm_plan.h picks one by sizes and alignment):
 //   k_gemm_big     256x256 tiles, M and N multiples of 256: direct global->LDS DMA, transposing LDS
 //                  reads for B, v_mfma_i32_32x32x32_i8.
 //   k_gemm_tile    tiles from 32x32 to 128x128 for every other shape and alignment, same operand
@@ -1334,7 +1334,7 @@ hipError_t x100_zero_i32_launch(int32_t *C, size_t n, hipStream_t s)
     return hipGetLastError();
 }
 
-// Kernel selection.  acc: C += A.B; otherwise C = A.B (the tile kernels never read C; the
+// The kernel of gemm_plan.h.  acc: C += A.B; otherwise C = A.B (the tile kernels never read C; the
 // split-K skinny kernels add partial sums with atomics, so their C is cleared first).  Returns the
 // HIP launch status.
 hipError_t x100_gemm_i8_launch(int M, int N, int K, const int8_t *A, const int8_t *B, int32_t *C,

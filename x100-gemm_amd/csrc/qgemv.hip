@@ -834,7 +834,7 @@ __global__ __launch_bounds__(NT) void k_q8_0(int M, int N, int K, int ngroups, c
 // The decode layer's output projection (one row, K 2049 to 4096), emitted here, ahead of the instances that the
 // launchers name, so that its place in the code object, and that of those after it, does not follow from which other
 // instances there are: without the 16 of 5 to 8 rows the layer at 4096 positions took 38.3-38.8 us instead of
-// 37.8-38.5, with this line 37.5-37.7 (four boxes; the machine code of every kernel is the same).
+// 37.8-38.5, with this line 37.4-37.7 (four cards; the machine code of every kernel is the same).
 template __global__ void k_q8_0<1, 32, 1, 4, 4, 256>(int M, int N, int K, int ngroups, const uint16_t *__restrict__ wd,
                                                      const int8_t *__restrict__ wq, const float *__restrict__ x,
                                                      float *__restrict__ y);
